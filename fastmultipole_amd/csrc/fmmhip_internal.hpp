@@ -127,6 +127,7 @@ struct Context {
     TreeScratch* tree_scratch = nullptr;
     ListScratch* list_scratch = nullptr;
     DBuf<int32_t> m2l_flags;    // pmax and success of the last M2L pass
+    DBuf<double> m2l_part;      // partial local expansions of long M2L lists (m2l_mx_gpu.hpp)
     DBuf<double> l2p_coef;      // per-leaf local-to-body coefficients of the last L2P pass
     DBuf<double> m2m_slot;      // per-child translated multipoles of one level of the upward pass
     DBuf<unsigned long long> p2p_queue;   // work counter of the persistent nearfield launch

@@ -118,16 +118,44 @@ static size_t mx_lds_bytes(int nw) {
     return sizeof(double) * (size_t)(mx_shared_doubles<CAP>() + nw * mx_wave_doubles<CAP, LH>());
 }
 
-// Persistent: every workgroup copies the tables into LDS once, then each wavefront takes whole target
-// boxes from a counter (flags[2]) and runs their interaction lists BP at a time; a box's local
-// expansion is summed in the wavefront's LDS and added to the target's expansion once, by the one
-// wavefront that owns the box (deterministic: the same sums in the same order on every run).
+// Work items. A target box's list entries are cut into chunks of S (the last one shorter), and a wavefront takes one
+// chunk at a time: with a wavefront per box the launch lasted as long as its longest list (45k ring at cap 20, 24,644
+// interactions in 1,400 boxes: 4.05 ms, when its 6,500 batches over 1024 wavefronts are 0.5 ms of work). Chunk c of
+// box b has slot l0 / S + b + c, l0 the box's first list entry: chunks of different boxes never share a slot
+// (ceil(len / S) <= floor(l1 / S) - floor(l0 / S) + 1), and the last slot is known on the host without a scan.
+// A box of one chunk is added to its target's expansion by the wavefront that holds it; the chunks of the others go to
+// `part` and k_m2l_mx_sum adds them in chunk order. S depends on the cap alone, never on the size of the problem, so a
+// box's sum is the same to the last bit whatever is evaluated beside it. S is a few batches: a chunk's partial
+// expansion (7.4 KB at cap 20) is written and read once per S interactions, 0.3 ms of the 1M ring's 30 ms.
+template <int CAP, bool LH>
+constexpr int mx_chunk() {
+    return (CAP <= 12 ? 2 : 4) * (LH ? 4 : 8);
+}
+__host__ __device__ inline int64_t mx_first_slot(int64_t l0, int64_t box, int S) { return l0 / S + box; }
+
+// the box whose slots hold slot w: the last one whose first slot is not above w (64 candidates per step)
+__device__ inline int mx_box_of(const int64_t* __restrict__ m2l_offsets, int n_boxes, int64_t w, int S, int lane) {
+    int lo = 0, len = n_boxes;
+    while (len > 1) {
+        const int step = (len + 63) >> 6;
+        const int k = lo + (lane + 1) * step;
+        const bool below = (lane + 1) * step < len && mx_first_slot(m2l_offsets[k], k, S) <= w;
+        const int moves = __popcll(__ballot(below));
+        lo += moves * step;
+        len = min(step, len - moves * step);
+    }
+    return __builtin_amdgcn_readfirstlane(lo);
+}
+
+// Persistent: every workgroup copies the tables into LDS once, then each wavefront takes chunks from a counter
+// (flags[2]) and runs their interactions BP at a time, summed in the wavefront's LDS.
 template <int CAP, bool LH, int NW, bool FULL>
 __global__ __launch_bounds__(64 * NW) void k_m2l_mx(const int32_t* __restrict__ m2l_targets,
                                                     const int64_t* __restrict__ m2l_offsets,
                                                     const int32_t* __restrict__ m2l_s, const Branch* __restrict__ tbr,
                                                     const Branch* __restrict__ sbr, const double* __restrict__ sex,
-                                                    double* __restrict__ tex, int n_boxes, int P, int PE, ErrParams E,
+                                                    double* __restrict__ tex, double* __restrict__ part, int n_boxes,
+                                                    int64_t n_slots, int P, int PE, ErrParams E,
                                                     const int32_t* __restrict__ perm, int32_t* __restrict__ orders,
                                                     int32_t* __restrict__ flags, int32_t* __restrict__ box_ok,
                                                     TablePtrs tb) {
@@ -167,11 +195,16 @@ __global__ __launch_bounds__(64 * NW) void k_m2l_mx(const int32_t* __restrict__ 
     const int64_t HE4 = 4 * (int64_t)nh(PE);
     const int lane = lane_id();
     int pmax = 0, okf = 1;
+    constexpr int S = mx_chunk<CAP, LH>();
     for (;;) {
-        int box = 0;
-        if (lane == 0) box = atomicAdd(flags + 2, 1);
-        box = __shfl(box, 0, 64);
-        if (box >= n_boxes) break;
+        int slot = 0;
+        if (lane == 0) slot = atomicAdd(flags + 2, 1);
+        slot = __builtin_amdgcn_readfirstlane(slot);
+        if (slot >= n_slots) break;
+        const int box = mx_box_of(m2l_offsets, n_boxes, slot, S, lane);
+        const int64_t lb = m2l_offsets[box], le = m2l_offsets[box + 1];
+        const int64_t l0 = lb + (slot - mx_first_slot(lb, box, S)) * S, l1 = min(le, l0 + S);
+        if (l0 >= le) continue;   // the box has one chunk fewer than slots
         for (int i = lane; i < NC * H; i += 64) W.acc[i] = 0.0;
         wave_sync();
         const int32_t it = m2l_targets[box];
@@ -187,7 +220,6 @@ __global__ __launch_bounds__(64 * NW) void k_m2l_mx(const int32_t* __restrict__ 
         X.P = P;
         X.kind = E.kind;
         X.BE = E.BE;
-        const int64_t l0 = m2l_offsets[box], l1 = m2l_offsets[box + 1];
         int okb = 1;
         for (int64_t b0 = l0; b0 < l1; b0 += BP) {
             const mx::Batch Bt{m2l_s, perm, (int)b0, (int)min((int64_t)BP, l1 - b0), orders};
@@ -198,13 +230,38 @@ __global__ __launch_bounds__(64 * NW) void k_m2l_mx(const int32_t* __restrict__ 
             okf = 0;
             if (box_ok && lane == 0) box_ok[box] = 0;
         }
-        double* dst = tex + (int64_t)it * HE4;
-        for (int i = lane; i < NC * nh(P); i += 64) dst[4 * (i / NC) + i % NC] += W.acc[i];
+        if (le - lb <= S) {
+            double* dst = tex + (int64_t)it * HE4;
+            for (int i = lane; i < NC * nh(P); i += 64) dst[4 * (i / NC) + i % NC] += W.acc[i];
+        } else {
+            double* dst = part + (int64_t)slot * (NC * nh(P));
+            for (int i = lane; i < NC * nh(P); i += 64) dst[i] = W.acc[i];
+        }
         wave_sync();
     }
     if (lane == 0) {
         atomicMax(flags, pmax);
         if (!okf) atomicAnd(flags + 1, 0);
+    }
+}
+
+// adds the chunks of each box of more than one, in chunk order, to its target's expansion
+template <int CAP, bool LH>
+__global__ __launch_bounds__(256) void k_m2l_mx_sum(const int32_t* __restrict__ m2l_targets,
+                                                    const int64_t* __restrict__ m2l_offsets, double* __restrict__ tex,
+                                                    const double* __restrict__ part, int P, int PE) {
+    constexpr int S = mx_chunk<CAP, LH>(), NC = LH ? 4 : 2;
+    const int box = blockIdx.x;
+    const int64_t l0 = m2l_offsets[box], l1 = m2l_offsets[box + 1];
+    if (l1 - l0 <= S) return;
+    const int64_t n = (l1 - l0 + S - 1) / S;
+    const int len = NC * nh(P);
+    const double* src = part + mx_first_slot(l0, box, S) * len;
+    double* dst = tex + (int64_t)m2l_targets[box] * (4 * (int64_t)nh(PE));
+    for (int i = threadIdx.x; i < len; i += 256) {
+        double v = src[i];
+        for (int64_t c = 1; c < n; ++c) v += src[c * len + i];
+        dst[4 * (i / NC) + i % NC] += v;
     }
 }
 
@@ -217,12 +274,18 @@ static void launch_m2l_mx(Context& C, int p, int pe, const Lists& Ls, const Tree
     int per_cu = 0;
     HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(kfn), 64 * NW, sh));
     if (!C.n_cu) HIP_CHECK(hipDeviceGetAttribute(&C.n_cu, hipDeviceAttributeMultiprocessorCount, C.device));
-    const int64_t want = (Ls.n_m2l_targets + NW - 1) / NW;
+    // one slot past the last box's first for each of its chunks (its list may end inside a chunk)
+    const int64_t slots = mx_first_slot(Ls.n_m2l, Ls.n_m2l_targets, mx_chunk<CAP, LH>());
+    const int64_t want = (slots + NW - 1) / NW;
+    C.m2l_part.resize((size_t)slots * ((LH ? 4 : 2) * nh(p)));
     const unsigned grid = (unsigned)std::max<int64_t>(1, std::min<int64_t>(want, (int64_t)std::max(per_cu, 1) * C.n_cu));
     kfn<<<grid, 64 * NW, sh, C.stream>>>(Ls.m2l_targets.data(), Ls.m2l_offsets.data(), Ls.m2l_s.data(), tt_dst.branches.data(),
-                                         st.branches.data(), st.expansions.data(), tt_dst.expansions.data(),
-                                         (int)Ls.n_m2l_targets, p, pe, E, perm, Ls.m2l_order.data(), flags,
+                                         st.branches.data(), st.expansions.data(), tt_dst.expansions.data(), C.m2l_part.data(),
+                                         (int)Ls.n_m2l_targets, slots, p, pe, E, perm, Ls.m2l_order.data(), flags,
                                          Ls.track_box_ok ? const_cast<int32_t*>(Ls.m2l_box_ok.data()) : nullptr, tb);
+    LAUNCH_CHECK();
+    k_m2l_mx_sum<CAP, LH><<<(unsigned)Ls.n_m2l_targets, 256, 0, C.stream>>>(Ls.m2l_targets.data(), Ls.m2l_offsets.data(),
+                                                                          tt_dst.expansions.data(), C.m2l_part.data(), p, pe);
     LAUNCH_CHECK();
 }
 

@@ -63,6 +63,7 @@ double footprint_bytes(const fmmhip_request& r) {
     double b = n * 8.0 * (fmmhip::data_per_body(r.kernel) + 3 + 13 + 16 + 24);
     b += 2.0 * branches * (sizeof(fmmhip::Branch) + 32.0 * H);
     b += branches * 400.0 * 16.0;
+    b += branches * 6.0 * 32.0 * H;   // partial expansions of the M2L's list chunks
     if (r.kind == FMMHIP_REQUEST_SOLVE) b += n * leaf * 8.0 * 30.0 + n * 8.0 * 40.0;
     return b;
 }
