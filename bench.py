@@ -506,12 +506,12 @@ def main():
                 "peak": PEAK_FP32_TFLOPS if main_form == "mixed" else PEAK_FP64_TFLOPS, "unit": "TFLOP/s",
                 "traffic": pmc_traffic(key)}
     # the error-controlled M2L: one persistent launch of the matrix-core engine at the order cap (the
-    # smallest instantiated cap >= pmax, specialised for order == cap); achieved = F(p) flops summed over
+    # smallest instantiated cap >= pmax); achieved = F(p) flops summed over
     # the interactions at the orders they used / the M2L phase time (the launch and the per-box ordering
     # sort before it)
     cap = next(c for c in (8, 12, 16, 20) if c >= args.pmax)
-    m2l_key = f"k_m2l_mx<{cap}, true, 4, {'true' if cap == args.pmax else 'false'}>"
-    roof_m2l = {"kernel": m2l_key + " (rotation-based M2L with Lamb-Helmholtz terms on v_mfma_f64_16x16x4f64, FP64; "
+    m2l_key = f"k_m2l_mx<{cap}, true, 4, true>"
+    roof_m2l = {"kernel": m2l_key + " (rotation-based M2L with Lamb-Helmholtz terms on v_mfma_f64_4x4x4_4b_f64, FP64; "
                                     "F(p) flop/interaction)",
                 "bound": "mfma", "achieved": round(m2l_tflops, 3), "peak": PEAK_FP64_TFLOPS, "unit": "TFLOP/s",
                 "traffic": pmc_traffic(m2l_key)}

@@ -1,30 +1,35 @@
-// Register-resident M2L on the matrix cores (v_mfma_f64_16x16x4f64, gfx950).
+// Register-resident M2L on the matrix cores (v_mfma_f64_4x4x4_4b_f64, gfx950).
 //
 // multipole_to_local! (src/translate.jl:519-550 fixed order, :555-1412 error-controlled) as rotate,
 // translate along z, Lamb-Helmholtz transform, rotate back, for BP interactions of one target box at once
-// per wavefront. The wavefront's 16 matrix columns are the real components of the BP interactions
-// ("slots"): NC = 4 with the Lamb-Helmholtz potential (phi re, phi im, chi re, chi im), NC = 2 without
-// (phi re, phi im), so BP = 16 / NC.
+// per wavefront. The wavefront's 16 matrix columns are the potentials of the BP interactions ("slots"):
+// NP = 2 with the Lamb-Helmholtz potential (phi, chi), NP = 1 without, so BP = 16 / NP. Real and imaginary
+// parts are two registers of the same lane.
 //
-// Register layout. A degree-n coefficient vector (rows m = 0..n, one column per component) is split by
+// Register layout. A degree-n coefficient vector (rows m = 0..n, one column per potential) is split by
 // the parity of m: the even part E holds m = 8e + 2q in register e of the lanes of quad q = lane / 16, the
-// odd part O holds m = 8o + 2q + 1, column = lane % 16. This is the layout in which the MFMA returns rows
-// i = 4r + q of a 16-row result when its rows are m = 2i (E) or m = 2i + 1 (O), and the layout in which
-// the next MFMA takes its B operand (lane l supplies B(l / 16, l % 16), so a result register r is the
-// K-block of rows 4r..4r+3). Products therefore chain with no data movement, and since a given m sits in
-// the same lane and register index for every degree, the z-translation L_j^m += F(j + k) M_k^m is a
-// lane-local multiply-add.
+// odd part O holds m = 8o + 2q + 1, column = lane % 16. A register is a group of four rows of one parity: the
+// K-block in which the 4x4x4 MFMA takes its B operand (lane l supplies B(l / 16, l % 16): four blocks of four
+// columns, every block with the same A), and the layout of the four rows that it returns. Products therefore
+// chain with no data movement, and since a given m sits in the same lane and register index for every degree, the
+// z-translation L_j^m += F(j + k) M_k^m is a lane-local multiply-add.
 //
 // Rotations. The y-rotation of degree n is the factorised form of the reference's Wigner matrices
 // (update_Ts!, src/rotate.jl:260-441, with the zeta / eta magnitudes of :625-1004):
-//   U = g_in(m') X,  S_E(v) = sum_{m' even} A(m', v) U_m',  S_O(v) = sum_{m' odd} A(m', v) U_m'
-//   P+ = (S_E - A(0, v) U_0) - S_O + s_v conj(S_E + S_O),  P- = (S_E - A(0, v) U_0) + S_O + s_v conj(S_E - S_O)
-//   Q+- = w_v (cos v b +- i sigma sin v b) P+-,  R_e = Q+ + Q-,  R_o = Q+ - Q-
-//   out_m = g_out(m) / 2 sum_v A(m, v) R_(parity of m)(v)
-// with A the degree-n pi/2 table (symmetric), s_v = (-1)^(n+v), w_0 = 1, w_v = 2. The two sums over m'
-// and the two sums over v are MFMA products whose A operand is the shared table (read from LDS with the
-// rows or columns of the other parity masked to zero); the combination is per element on the vector ALU
-// (the re / im partner of a component is the neighbouring lane, reached by DPP).
+//   U = g_in(m') X,  S_E(v) = A(0, v) U_0 / 2 + sum_{m' even > 0} A(m', v) U_m',  S_O(v) = sum_{m' odd} A(m', v) U_m'
+//   n + v even:  R_e = cos Re S_E + sigma sin Im S_O           (real),
+//                R_o = sigma sin Re S_E - cos Im S_O           (imaginary)
+//   n + v odd:   R_e = cos Im S_E - sigma sin Re S_O           (imaginary),
+//                R_o = -(cos Re S_O + sigma sin Im S_E)        (real),    cos, sin of v beta
+//   out_m = 4 g_out(m) sum_v w_v A(m, v) R_(parity of m)(v),  w_0 = 1/2, else 1
+// with A the degree-n pi/2 table (symmetric; A(0, v) = 0 for n + v odd). So for every v one of the two sums is needed
+// per real or imaginary part, not both: with real and imaginary parts in registers of their own and the v of one
+// parity in a register, the products that are not needed are not formed, and the combination is two multiplies and
+// two multiply-adds in the lane. (Components in neighbouring columns, sums over m' and v in 16x16x4 products and the
+// combination masked per element over DPP exchanges took 31,000 instructions per 4 interactions at order 20.) The
+// number of 4x4x4 products of a degree is 2 (KE + KO)^2 for 16 complex columns, each at a quarter of a 16x16x4's 64
+// cycles, and their FP64 units are those of the vector ALU: the two do not overlap (measured: a product and a
+// multiply-add take the sum of their times), so both counts matter.
 //
 // z-translation, streamed by degree. The reference forms L_n^m = sum_{k=m}^{P} F(n + k) M_k^m with
 // F(j) = j! / t^(j+1) after the whole rotated multipole exists. Here degree k of the multipole is
@@ -59,8 +64,6 @@ namespace mx {
 constexpr int mnh(int p) { return p < 0 ? 0 : ((p + 1) * (p + 2)) >> 1; }
 constexpr int KE(int n) { return (n / 2 + 4) / 4; }          // registers of the even part of degree n
 constexpr int KO(int n) { return ((n + 1) / 2 + 3) / 4; }    // registers of the odd part
-constexpr int KB(int n) { return (n + 4) / 4; }              // 4-row blocks of rows 0..n
-constexpr int TE(int n) { return (n + 16) / 16; }            // 16-row tiles of rows 0..n
 constexpr int LOFF(int n) { return n <= 0 ? 0 : LOFF(n - 1) + KE(n - 1) + KO(n - 1); }   // degree n in L
 constexpr int NLREG(int cap) { return LOFF(cap + 1); }
 template <int n>
@@ -70,6 +73,9 @@ struct LO {   // LOFF(n) as a constant (register arrays need compile-time indice
 constexpr int AST(int n) { return (n + 2) & ~1; }            // row length of the dense pi/2 table of degree n
 constexpr int ABASE(int n) { return (n * (n + 1) * (2 * n + 1)) / 6 + ((n + 1) / 2) * ((n + 1) / 2); }
 constexpr int ALEN(int cap) { return ABASE(cap + 1); }
+// zero-padded pi/2 table: degree n as (KE + KO)^2 blocks of 4x4 at PBASE(n), rows and columns by parity (E groups, then O)
+constexpr int PBASE(int n) { return n <= 0 ? 0 : PBASE(n - 1) + 16 * (KE(n - 1) + KO(n - 1)) * (KE(n - 1) + KO(n - 1)); }
+constexpr int PLEN(int cap) { return PBASE(cap + 1); }
 constexpr int imin(int a, int b) { return a < b ? a : b; }
 constexpr int imax(int a, int b) { return a > b ? a : b; }
 
@@ -81,9 +87,32 @@ MX_FN void sfor(F&& f) {
     }
 }
 
+// d += A B on four blocks of 4x4x4: lane l supplies A(l % 4, l / 16) (the same in every block), B(l / 16, l % 16) and
+// holds D(l / 16, l % 16). A backend without the instruction takes the first four rows of the 16x16x4 product.
+template <class B, class = void>
+struct Prod {
+    MX_FN static void add(const typename B::V& a, const typename B::V& b, typename B::V& d) {
+        typename B::V4 t = B::zero4();
+        B::set4(t, 0, d);
+        B::mfma(a, b, t);
+        d = B::get4(t, 0);
+    }
+};
+template <class B>
+struct Prod<B, std::void_t<decltype(&B::mfma4)>> {
+    MX_FN static void add(const typename B::V& a, const typename B::V& b, typename B::V& d) { d = B::mfma4(a, b, d); }
+};
+
+// A backend with `padded` holds the pi/2 tables in the zero-padded form. Rows and columns past the degree are then zero in
+// every product, so no row of a rotation needs a mask; in the dense form such entries belong to other rows.
+template <class B, class = void>
+struct Padded : std::false_type {};
+template <class B>
+struct Padded<B, std::void_t<typename B::padded>> : std::true_type {};
+
 // Shared tables (LDS on the GPU), for degrees 0..CAP; per (n, m) tables are indexed mnh(n - 1) + m.
 struct Tabs {
-    const double* A;     // dense pi/2 tables: degree n at ABASE(n), row-major, rows of AST(n)
+    const double* A;     // dense pi/2 tables: degree n at ABASE(n), row-major, rows of AST(n); or the padded form (PBASE)
     const double* zin;   // zeta input scale (multipole rotation)
     const double* zoh;   // half the zeta output scale
     const double* ein;   // eta input scale (local rotation)
@@ -96,8 +125,8 @@ struct Tabs {
 
 // per-wavefront scratch
 struct Wave {
-    double* eim;   // BP x (CAP + 1) x 2: e^{i m alpha} of each slot
-    double* cs;    // BP x (CAP + 1) x 2: cos / sin (v beta) of each slot
+    double* eim;   // BP x (CAP + 1) x 2: 8 e^{i m alpha} of each slot (the 8 is the rotation's 4 and g_out's halves)
+    double* cs;    // BP x (CAP + 1) x 2: w_v cos / sin (v beta) of each slot
     double* acc;   // mnh(CAP) x NC: the target box's local expansion, summed over the wave's interactions
     double* F;     // BP x (2 CAP + 1): z-translation factors j! / t^(j+1) of each slot
 };
@@ -121,16 +150,18 @@ struct Box {
     int BE;         // the order settles at the passing degree (1) or one below (0)
 };
 
-template <class B, int CAP, bool LH, bool FULL = false>
+// EK: 0 fixed orders only, 1 error-controlled only, -1 either (Box::kind says which)
+template <class B, int CAP, bool LH, int EK = -1>
 struct Engine {
     using V = typename B::V;
     using I = typename B::I;
     using M = typename B::M;
-    using V4 = typename B::V4;
     using PV = typename B::PV;
-    static constexpr int NC = LH ? 4 : 2;
-    static constexpr int BP = 16 / NC;
-    static constexpr int NL = NLREG(CAP);
+    static constexpr int NP = LH ? 2 : 1;    // potentials
+    static constexpr int NC = 2 * NP;        // real components per coefficient
+    static constexpr int BP = 16 / NP;
+    static constexpr bool PAD = Padded<B>::value;
+    static constexpr int NL = NLREG(CAP);    // registers of the local expansion, per real or imaginary part
     static constexpr int NS = CAP + 1;   // slot-table entries
     static constexpr int NF = 2 * CAP + 1;   // translation factors per slot
     static constexpr int NX = KE(CAP) + KO(CAP);   // registers of one degree
@@ -144,10 +175,10 @@ struct Engine {
         return B::sel(same, mn, V(0.0));
     }
 
-    // list index of slot `slot` of the batch
+    // list index of slot `slot` of the batch (of its first slot for an empty one)
     MX_FN static I entry(const Batch& Bt, I slot, M ok) {
         const I k = B::seli(ok, slot, I(0)) + Bt.b0;
-        return Bt.perm ? B::gldi(Bt.perm, k, ok) : k;
+        return Bt.perm ? B::gldi(Bt.perm, k, M(true)) : k;
     }
 
     // translation vector target centre - source centre of source branch js (benign values for empty slots)
@@ -192,7 +223,8 @@ struct Engine {
         V cp, sp, cb, sb;
         const V r = angles(dx, dy, dz, cp, sp, cb, sb);
         const V ot = 1.0 / r;
-        V er = 1.0, ei = 0.0, c = 1.0, s = 0.0, f = ot;
+        // an empty slot's phases are zero: its multipole and its local expansion are then zero in every degree
+        V er = B::sel(vT, V(8.0), V(0.0)), ei = 0.0, c = 1.0, s = 0.0, f = ot;
         auto step = [&](M st, int x) {
             const V t = er;
             const V ner = er * cp - ei * sp;
@@ -224,136 +256,127 @@ struct Engine {
             const I idx = B::seli(okk, (sT * NS + k) * 2, I(0));
             B::lds_st(W.eim, idx, er, okk);
             B::lds_st(W.eim, idx + 1, ei, okk);
-            B::lds_st(W.cs, idx, c, okk);
+            if constexpr (h == 0) B::lds_st(W.cs, idx, B::sel(kT == 0, V(0.5), c), okk);
+            else B::lds_st(W.cs, idx, c, okk);
             B::lds_st(W.cs, idx + 1, s, okk);
             B::lds_st(W.F, B::seli(okf, sT * NF + k, I(0)), f, okf);
         });
         B::wsync();
     }
 
-    // Lane constants of the rotation's combination step
-    struct RotLane {
-        I c, q, s;
-        V sq;    // (-1)^q, negated on imaginary lanes: (-1)^(n+v) conj() for rows v = 16 t + 4 r + q
-        V nj;    // +1 on imaginary lanes, -1 on real ones: the i of a complex product
-        V w0;    // w_v of row v = q (1 for v = 0, else 2)
-    };
-
-    // One rotation of degree n (compile-time) of the coefficient vector u (E / O registers, input scale
-    // applied, rows m > n zero): out = g_out / 2 * A . R(A^T . u). sigma = +1 multipole (zeta), -1 local
-    // (eta). The A operands are read unmasked: entries outside the degree's table multiply zero rows of u
-    // (first products) or rows of R that are set to zero (second products), or land in output rows m > n,
-    // which are discarded; every address stays inside the shared tables.
+    // One rotation of degree n (compile-time) of the coefficient vector u (input scale applied, row 0 halved, rows
+    // m > n zero): out as in the header, without the factor 4 w (in the slot tables) and with rows m > n zero. sigma = +1
+    // multipole (zeta), -1 local (eta). In the dense form the A operands are read unmasked: entries outside the degree's
+    // table multiply zero rows of u (first products) or rows of R that are set to zero (second products), or land in
+    // output rows m > n, which are discarded. In the padded form these rows may hold any finite value.
     template <int n>
-    MX_FN static void rotate(const Tabs& T, const Wave& W, const double* gout, double sigma, const RotLane& RL,
-                             const V (&uE)[imax(KE(n), 1)], const V (&uO)[imax(KO(n), 1)], V (&oE)[imax(KE(n), 1)],
-                             V (&oO)[imax(KO(n), 1)]) {
-        constexpr int ke = KE(n), ko = KO(n), te = TE(n), kb = KB(n), st = AST(n), ab = ABASE(n);
-        const I c = RL.c, q = RL.q, s = RL.s;
-        V4 SE[te], SO[te];
-        sfor<0, te>([&](auto TT) {
-            constexpr int t = decltype(TT)::value;
-            SE[t] = B::zero4();
-            SO[t] = B::zero4();
-        });
-        // first products: rows v = 16 t + (lane % 16), K = the even (odd) rows m' of u
-        const I lo1 = q * (2 * st) + c;
-        sfor<0, te>([&](auto TT) {
-            constexpr int t = decltype(TT)::value;
-            sfor<0, ke>([&](auto EE) {
-                constexpr int e = decltype(EE)::value;
-                B::mfma(B::lds(T.A, lo1 + (ab + 8 * e * st + 16 * t)), uE[e], SE[t]);
-            });
-            sfor<0, ko>([&](auto OO) {
-                constexpr int o = decltype(OO)::value;
-                B::mfma(B::lds(T.A, lo1 + (ab + (8 * o + 1) * st + 16 * t)), uO[o], SO[t]);
-            });
-        });
-        // combination, per element (rows v of the first products)
-        const V U0 = B::bperm(uE[0], c);
+    MX_FN static void rotate(const Tabs& T, const Wave& W, const double* gout, double sigma, I c, I q, I s,
+                             const V (&uEr)[imax(KE(n), 1)], const V (&uEi)[imax(KE(n), 1)], const V (&uOr)[imax(KO(n), 1)],
+                             const V (&uOi)[imax(KO(n), 1)], V (&oEr)[imax(KE(n), 1)], V (&oEi)[imax(KE(n), 1)],
+                             V (&oOr)[imax(KO(n), 1)], V (&oOi)[imax(KO(n), 1)]) {
+        constexpr int ke = KE(n), ko = KO(n), st = AST(n), ab = ABASE(n);
+        const I q2 = q * 2, i2 = (c & 3) * 2;
+        const I lo = i2 * st + q2;
+        // A block of rows 8 r + pr + 2 (lane % 4) and columns 8 k + pk + 2 (lane / 16)
+        auto blk = [&](auto R, auto PR, auto KK, auto PK) {
+            constexpr int r0 = 8 * decltype(R)::value + decltype(PR)::value, k0 = 8 * decltype(KK)::value + decltype(PK)::value;
+            if constexpr (PAD) {
+                constexpr int rq = decltype(R)::value + (decltype(PR)::value ? ke : 0);
+                constexpr int kq = decltype(KK)::value + (decltype(PK)::value ? ke : 0);
+                return B::lds(T.A, i2 * 2 + q + (PBASE(n) + (rq * (ke + ko) + kq) * 16));
+            } else if constexpr (ab + (r0 + 6) * st + k0 + 6 < ALEN(CAP)) return B::lds(T.A, lo + (ab + r0 * st + k0));
+            else return B::lds(T.A, B::mini(i2 + r0, n) * st + B::mini(q2 + k0, n) + ab);
+        };
+        using C0 = std::integral_constant<int, 0>;
+        using C1 = std::integral_constant<int, 1>;
         const I sb = s * (NS * 2);
-        sfor<0, te>([&](auto TT) {
-            constexpr int t = decltype(TT)::value;
-            sfor<0, 4>([&](auto RR) {
-                constexpr int r = decltype(RR)::value;
-                constexpr int v0 = 16 * t + 4 * r;
-                if constexpr (v0 <= n) {
-                    const I v = q + v0;
-                    const V se = B::get4(SE[t], r), so = B::get4(SO[t], r);
-                    const V a00 = B::lds(T.A, q + (ab + v0));
-                    const I ci = sb + B::mini(v, n) * 2;
-                    const V cv = B::lds(W.cs, ci), sv = B::lds(W.cs, ci + 1);
-                    V cc, sn;
-                    if constexpr (v0 == 0) {
-                        cc = RL.w0 * cv;
-                        sn = RL.w0 * sigma * sv;
-                    } else {
-                        cc = 2.0 * cv;
-                        sn = (2.0 * sigma) * sv;
-                    }
-                    const V sgc = (n & 1) ? -RL.sq : RL.sq;
-                    const V D = se - a00 * U0;
-                    const V Pp = (D - so) + sgc * (se + so);
-                    const V Pm = (D + so) + sgc * (se - so);
-                    const V snj = sn * RL.nj;
-                    const V Qp = cc * Pp + snj * B::perm1(Pp);
-                    const V Qm = cc * Pm - snj * B::perm1(Pm);
-                    if constexpr (v0 + 3 <= n) {
-                        B::set4(SE[t], r, Qp + Qm);   // R_e
-                        B::set4(SO[t], r, Qp - Qm);   // R_o
-                    } else {
-                        const M okv = v <= n;
-                        B::set4(SE[t], r, B::sel(okv, Qp + Qm, V(0.0)));
-                        B::set4(SO[t], r, B::sel(okv, Qp - Qm, V(0.0)));
-                    }
-                } else {
-                    B::set4(SE[t], r, V(0.0));
-                    B::set4(SO[t], r, V(0.0));
-                }
-            });
-        });
-        // second products: rows m = 2 (lane % 16) (+1), K = rows v
-        V4 PE = B::zero4(), PO = B::zero4();
-        const I lo2 = q * st + c * 2;
-        sfor<0, kb>([&](auto BB) {
-            constexpr int b = decltype(BB)::value;
-            B::mfma(B::lds(T.A, lo2 + (ab + 4 * b * st)), B::get4(SE[b / 4], b % 4), PE);
-            B::mfma(B::lds(T.A, lo2 + (ab + 4 * b * st + 1)), B::get4(SO[b / 4], b % 4), PO);
-        });
-        auto out = [&](auto par, auto RI, const V4& Pv, V& o) {
-            constexpr int pr = decltype(par)::value, ri = decltype(RI)::value;
-            constexpr int m0 = 8 * ri + pr;
-            const I m = q * 2 + m0;
-            if constexpr (m0 + 6 <= n) {
-                o = B::lds(gout, m + mnh(n - 1)) * B::get4(Pv, ri);
+        auto okrow = [&](auto par, auto RI) { return q2 + (8 * decltype(RI)::value + decltype(par)::value) <= n; };
+        sfor<0, ke>([&](auto AA) { oEr[decltype(AA)::value] = V(0.0); oEi[decltype(AA)::value] = V(0.0); });
+        sfor<0, imax(ko, 1)>([&](auto AA) { oOr[decltype(AA)::value] = V(0.0); oOi[decltype(AA)::value] = V(0.0); });
+        // the v of one register (parity par): first products, combination, second products
+        auto half = [&](auto par, auto VI) {
+            constexpr int pv = decltype(par)::value, vi = decltype(VI)::value, v0 = 8 * vi + pv;
+            constexpr bool even = ((n + pv) & 1) == 0;   // n + v even
+            V se = V(0.0), so = V(0.0);   // the needed parts of S_E and S_O
+            sfor<0, ke>([&](auto EE) { Prod<B>::add(blk(VI, par, EE, C0()), even ? uEr[decltype(EE)::value] : uEi[decltype(EE)::value], se); });
+            sfor<0, ko>([&](auto OO) { Prod<B>::add(blk(VI, par, OO, C1()), even ? uOi[decltype(OO)::value] : uOr[decltype(OO)::value], so); });
+            const I vr = (PAD || v0 + 6 <= n) ? q2 + v0 : B::mini(q2 + v0, n);
+            const I ci = sb + vr * 2;
+            const V cv = B::lds(W.cs, ci), sv = B::lds(W.cs, ci + 1) * sigma;
+            V re, ro;
+            if constexpr (even) {
+                re = B::fma(sv, so, cv * se);
+                ro = B::fma(-cv, so, sv * se);
             } else {
-                const M ok = m <= n;
-                o = B::sel(ok, B::lds(gout, B::mini(m, n) + mnh(n - 1)) * B::get4(Pv, ri), V(0.0));
+                re = B::fma(-sv, so, cv * se);
+                ro = -B::fma(cv, so, sv * se);
+            }
+            if constexpr (!PAD && v0 + 6 > n) {
+                const M ok = okrow(par, VI);
+                re = B::sel(ok, re, V(0.0));
+                ro = B::sel(ok, ro, V(0.0));
+            }
+            sfor<0, ke>([&](auto AA) {
+                constexpr int a = decltype(AA)::value;
+                Prod<B>::add(blk(AA, C0(), VI, par), re, even ? oEr[a] : oEi[a]);
+            });
+            sfor<0, ko>([&](auto AA) {
+                constexpr int a = decltype(AA)::value;
+                Prod<B>::add(blk(AA, C1(), VI, par), ro, even ? oOi[a] : oOr[a]);
+            });
+        };
+        sfor<0, ke>([&](auto VI) { half(C0(), VI); });
+        sfor<0, ko>([&](auto VI) { half(C1(), VI); });
+        auto out = [&](auto par, auto RI, V& xr, V& xi) {
+            constexpr int m0 = 8 * decltype(RI)::value + decltype(par)::value;
+            if constexpr (PAD || m0 + 6 <= n) {
+                const V g = B::lds(gout, q2 + (m0 + mnh(n - 1)));
+                xr = g * xr;
+                xi = g * xi;
+            } else {
+                const M ok = q2 + m0 <= n;
+                const V g = B::lds(gout, B::mini(q2 + m0, n) + mnh(n - 1));
+                xr = B::sel(ok, g * xr, V(0.0));
+                xi = B::sel(ok, g * xi, V(0.0));
             }
         };
-        sfor<0, ke>([&](auto EE) { out(std::integral_constant<int, 0>(), EE, PE, oE[decltype(EE)::value]); });
-        sfor<0, ko>([&](auto OO) { out(std::integral_constant<int, 1>(), OO, PO, oO[decltype(OO)::value]); });
+        sfor<0, ke>([&](auto EE) { out(C0(), EE, oEr[decltype(EE)::value], oEi[decltype(EE)::value]); });
+        sfor<0, ko>([&](auto OO) { out(C1(), OO, oOr[decltype(OO)::value], oOi[decltype(OO)::value]); });
     }
 
-    // the source coefficients of degree n for this lane's rows (E registers, then O), zero for rows m > n
-    // and for empty slots
+    // the source coefficients of degree n for this lane's rows (E registers, then O); rows m > n are zero, or row n's in
+    // the padded form
     template <int n>
-    MX_FN static void fetch(const PV& src, I q, I comp, M valid, V (&xn)[NX]) {
-        auto one = [&](auto par, auto RI, V& x) {
-            constexpr int pr = decltype(par)::value, ri = decltype(RI)::value;
-            constexpr int m0 = 8 * ri + pr;
-            const I m = q * 2 + m0;
-            const M ok = (m0 + 6 <= n) ? valid : (valid && (m <= n));
-            const I mi = (m0 + 6 <= n) ? m : B::mini(m, n);
-            x = B::gldp(src, (mi + mnh(n - 1)) * 4 + comp, ok);
+    MX_FN static void fetch(const PV& src, I q, I pot, V (&xr)[NX], V (&xi)[NX]) {
+        auto one = [&](auto par, auto RI, V& r, V& i) {
+            constexpr int m0 = 8 * decltype(RI)::value + decltype(par)::value;
+            const I at = (q * 2) * 4 + pot * 2;
+            constexpr int k0 = (m0 + mnh(n - 1)) * 4;
+            if constexpr (PAD && m0 + 6 > n) {
+                const I last = B::mini(q * 2 + m0, n) * 4 + pot * 2;
+                r = B::gldp(src, last + mnh(n - 1) * 4, M(true));
+                i = B::gldp(src, last + (mnh(n - 1) * 4 + 1), M(true));
+            } else if constexpr (m0 + 6 <= n) {
+                r = B::gldp(src, at + k0, M(true));
+                i = B::gldp(src, at + (k0 + 1), M(true));
+            } else {
+                const M ok = q * 2 + m0 <= n;
+                r = B::gldp(src, at + k0, ok);
+                i = B::gldp(src, at + (k0 + 1), ok);
+            }
         };
-        sfor<0, KE(n)>([&](auto EE) { one(std::integral_constant<int, 0>(), EE, xn[decltype(EE)::value]); });
-        sfor<0, KO(n)>([&](auto OO) { one(std::integral_constant<int, 1>(), OO, xn[KE(n) + decltype(OO)::value]); });
+        sfor<0, KE(n)>([&](auto EE) { one(std::integral_constant<int, 0>(), EE, xr[decltype(EE)::value], xi[decltype(EE)::value]); });
+        sfor<0, KO(n)>([&](auto OO) {
+            one(std::integral_constant<int, 1>(), OO, xr[KE(n) + decltype(OO)::value], xi[KE(n) + decltype(OO)::value]);
+        });
     }
 
-    // value of component j of this lane's slot, from the same lane quad
-    template <int j>
-    MX_FN static V comp_of(V x) { return B::template qbcast<NC, j>(x); }
+    // phi's and chi's value of a column, in both of the slot's columns
+    MX_FN static V phi_of(V x) {
+        if constexpr (LH) return B::template qbcast<2, 0>(x);
+        else return x;
+    }
+    MX_FN static V chi_of(V x) { return B::template qbcast<2, 1>(x); }
 
     // One batch of interactions of one target box: their local expansions are added to W.acc and their
     // orders written to Bt.orders. pmax / ok collect the largest order and whether every tolerance was met.
@@ -362,37 +385,31 @@ struct Engine {
         slot_tables(X, W, Bt, sbr, br_stride, sc_off);
         const I l0 = B::lane();
         const I c0 = l0 & 15, q0 = l0 >> 4;
-        const I c = c0, q = q0, s = c / NC, comp = c % NC, pot = comp >> 1;
-        const M isIm = (comp & 1) != 0;
-        const M valid = s < Bt.nb;
-        const int P = FULL ? CAP : X.P;   // FULL: the launch's order is the engine's cap
-        const bool err = X.kind != 0;
+        const I s0 = LH ? (c0 >> 1) & 7 : c0, pot0 = LH ? c0 & 1 : I(0);
+        const M valid = s0 < Bt.nb;
+        const int P = X.P;
+        const bool err = EK < 0 ? X.kind != 0 : EK != 0;
 
-        const I li = entry(Bt, s, valid);
-        const I js = B::gldi(Bt.m2l_s, li, valid);
+        // an empty slot reads the batch's first interaction; its phases are zero (slot_tables)
+        const I li = entry(Bt, s0, valid);
+        const I js = B::gldi(Bt.m2l_s, li, M(true));
         V dx, dy, dz;
         geometry(X, js, valid, sbr, br_stride, sc_off, dx, dy, dz);
         const V r = B::sqrt(dx * dx + dy * dy + dz * dz);
-        const V d0 = md1(dx, -X.tbox[0], X.tbox[0]), d1 = md1(dy, -X.tbox[1], X.tbox[1]), d2 = md1(dz, -X.tbox[2], X.tbox[2]);
-        const V r_mp = B::sqrt(d0 * d0 + d1 * d1 + d2 * d2);
-        const V rmi = 1.0 / r_mp;
         const PV src = B::ptr(sex, js, HE4);
-        const V cj = B::sel(isIm, V(-1.0), V(1.0));
-        const V phi_sign = B::sel(comp == 0, V(-1.0), B::sel(comp == 1, V(1.0), V(0.0)));   // Lamb-Helmholtz phi term
-        const M chi_lane = pot == 1;
-        RotLane RL0;
-        RL0.c = c;
-        RL0.q = q;
-        RL0.s = s;
-        RL0.sq = B::sel((q & 1) != 0, -cj, cj);
-        RL0.nj = -cj;
-        RL0.w0 = B::sel(q == 0, V(1.0), V(2.0));
+        const M chi_lane = pot0 == 1;
+        V r_mp = V(1.0), rmi = V(1.0);
+        if (err) {
+            const V d0 = md1(dx, -X.tbox[0], X.tbox[0]), d1 = md1(dy, -X.tbox[1], X.tbox[1]), d2 = md1(dz, -X.tbox[2], X.tbox[2]);
+            r_mp = B::sqrt(d0 * d0 + d1 * d1 + d2 * d2);
+            rmi = 1.0 / r_mp;
+        }
 
-        V L[NL];
-        sfor<0, NL>([&](auto II) { L[decltype(II)::value] = V(0.0); });
+        V Lr[NL], Li[NL];
+        sfor<0, NL>([&](auto II) { Lr[decltype(II)::value] = V(0.0); Li[decltype(II)::value] = V(0.0); });
         // degree k's source coefficients are loaded during degree k - 1 (their HBM latency hidden)
-        V xn[NX];
-        fetch<0>(src, q, comp, valid, xn);
+        V xnr[NX], xni[NX];
+        fetch<0>(src, q0, pot0, xnr, xni);
         M active = valid;
         M succ = valid && !err;
         I Pl = I(P);
@@ -410,97 +427,94 @@ struct Engine {
             constexpr int ke = KE(k), ko = KO(k), ke1 = imax(ke, 1), ko1 = imax(ko, 1);
             // lane indices made opaque per degree: their derived addresses and masks are recomputed here
             // instead of being hoisted (one register each for the whole kernel)
-            const I c = B::opaque(c0), q = B::opaque(q0), s = c / NC, comp = c % NC, pot = comp >> 1;
-            const I fb = s * NF, sb2 = s * (NS * 2);
-            RotLane RL = RL0;
-            RL.c = c;
-            RL.q = q;
-            RL.s = s;
+            const I c = B::opaque(c0) & 15, q = B::opaque(q0) & 3;
+            const I s = LH ? c >> 1 : c, pot = LH ? c & 1 : I(0);
+            const I fb = s * NF, sb2 = s * (NS * 2), q2 = q * 2;
             // ---- degree k of the source multipoles: power terms, z-rotation, input scale
-            V uE[ke1], uO[ko1], ME[ke1], MO[ko1];
-            V xc[NX];
-            sfor<0, ke + ko>([&](auto II) { xc[decltype(II)::value] = xn[decltype(II)::value]; });
+            V uEr[ke1], uEi[ke1], uOr[ko1], uOi[ko1], MEr[ke1], MEi[ke1], MOr[ko1], MOi[ko1];
+            V xcr[NX], xci[NX];
+            sfor<0, ke + ko>([&](auto II) {
+                xcr[decltype(II)::value] = xnr[decltype(II)::value];
+                xci[decltype(II)::value] = xni[decltype(II)::value];
+            });
             if constexpr (k + 1 <= CAP) {
-                if (FULL || k + 1 <= P) fetch<k + 1>(src, q, comp, valid, xn);
+                if (k + 1 <= P) fetch<k + 1>(src, q, pot, xnr, xni);
             }
             V pw_t = V(0.0);
-            const bool power = X.kind >= 2;
-            auto load = [&](auto par, auto RI, V& u) {
-                constexpr int pr = decltype(par)::value, ri = decltype(RI)::value;
-                constexpr int m0 = 8 * ri + pr;
-                const I m = q * 2 + m0;
-                const I mi = (m0 + 6 <= k) ? m : B::mini(m, k);
-                const V x = xc[(pr ? ke : 0) + ri];
+            const bool power = err && X.kind >= 2;
+            auto load = [&](auto par, auto RI, V& ur, V& ui) {
+                constexpr int pr = decltype(par)::value, ri = decltype(RI)::value, m0 = 8 * ri + pr;
+                const I mi = (PAD || m0 + 6 <= k) ? q2 + m0 : B::mini(q2 + m0, k);
+                const V xr = xcr[(pr ? ke : 0) + ri], xi = xci[(pr ? ke : 0) + ri];
                 if (power) {
-                    const V nt = B::lds(T.Mt, mi + mnh(k - 1));
-                    const V x2 = x * x;
-                    pw_t = pw_t + (x2 + B::perm1(x2)) * nt * nt;
+                    V nt = B::lds(T.Mt, mi + mnh(k - 1));
+                    if constexpr (PAD && m0 + 6 > k) nt = B::sel(q2 + m0 <= k, nt, V(0.0));
+                    pw_t = B::fma(B::fma(xr, xr, xi * xi) * nt, nt, pw_t);
                 }
                 const I ei = sb2 + mi * 2;
                 const V er = B::lds(W.eim, ei), eimg = B::lds(W.eim, ei + 1);
-                const V y = x * er + RL.nj * B::perm1(x) * eimg;
-                u = B::lds(T.zin, mi + mnh(k - 1)) * y;
+                const V g = B::lds(T.zin, mi + mnh(k - 1));
+                ur = g * B::fma(xr, er, -(xi * eimg));
+                ui = g * B::fma(xi, er, xr * eimg);
+                if constexpr (m0 == 0) ur = ur * B::sel(q == 0, V(0.5), V(1.0));   // half of row 0 (ui's multiplies A(0, v) = 0)
             };
-            sfor<0, ke>([&](auto EE) { load(std::integral_constant<int, 0>(), EE, uE[decltype(EE)::value]); });
-            sfor<0, ko>([&](auto OO) { load(std::integral_constant<int, 1>(), OO, uO[decltype(OO)::value]); });
-            if constexpr (ko == 0) uO[0] = V(0.0);
+            sfor<0, ke>([&](auto EE) { load(std::integral_constant<int, 0>(), EE, uEr[decltype(EE)::value], uEi[decltype(EE)::value]); });
+            sfor<0, ko>([&](auto OO) { load(std::integral_constant<int, 1>(), OO, uOr[decltype(OO)::value], uOi[decltype(OO)::value]); });
+            if constexpr (ko == 0) { uOr[0] = V(0.0); uOi[0] = V(0.0); }
             V pw_phi = V(0.0), pw_chi = V(0.0);
             if (power) {
-                const V t = B::quadsum(pw_t);
-                if (LH) {
-                    const V o = B::perm2(t);
-                    pw_phi = B::sqrt(B::sel(pot == 0, t, o));
-                    pw_chi = B::sqrt(B::sel(pot == 1, t, o));
-                } else {
-                    pw_phi = B::sqrt(t);
-                }
+                const V t = B::sqrt(B::quadsum(pw_t));
+                pw_phi = phi_of(t);
+                if constexpr (LH) pw_chi = chi_of(t);
             }
             // ---- y-rotation of degree k (rotate_multipole_y!, zeta magnitudes)
-            rotate<k>(T, W, T.zoh, 1.0, RL, uE, uO, ME, MO);
+            rotate<k>(T, W, T.zoh, 1.0, c, q, s, uEr, uEi, uOr, uOi, MEr, MEi, MOr, MOi);
             // ---- L_k += F(2k) M_k
             {
-                const V fac = B::sel(active, B::lds(W.F, fb + 2 * k), V(0.0));
+                V fac = B::lds(W.F, fb + 2 * k);
+                if (err) fac = B::sel(active, fac, V(0.0));
                 sfor<0, ke>([&](auto EE) {
                     constexpr int e = decltype(EE)::value;
-                    L[LO<k>::v + e] = B::fma(fac, ME[e], L[LO<k>::v + e]);
+                    Lr[LO<k>::v + e] = B::fma(fac, MEr[e], Lr[LO<k>::v + e]);
+                    Li[LO<k>::v + e] = B::fma(fac, MEi[e], Li[LO<k>::v + e]);
                 });
                 sfor<0, ko>([&](auto OO) {
                     constexpr int o = decltype(OO)::value;
-                    L[LO<k>::v + ke + o] = B::fma(fac, MO[o], L[LO<k>::v + ke + o]);
+                    Lr[LO<k>::v + ke + o] = B::fma(fac, MOr[o], Lr[LO<k>::v + ke + o]);
+                    Li[LO<k>::v + ke + o] = B::fma(fac, MOi[o], Li[LO<k>::v + ke + o]);
                 });
             }
             // ---- order tests of degree k. Uniform factors are formed once per degree from reciprocal
             // tables (reordered products: test values agree with the reference's to a few ulps), and the
             // local part is skipped when no active interaction's multipole part is within the tolerance
             // (the reference evaluates it only then).
-            M pass = M(false);
-            if constexpr (k >= 1) {
-                if (err) {
+            if (err) {
+                M pass = M(false);
+                if constexpr (k >= 1) {
                     constexpr double ik = 1.0 / k, ik1 = 1.0 / (k + 1);
                     const double nm1_f_inv = T.tf[2 * k], np1_f = T.tf[2 * k + 1];
                     V eps_mp, eps_l = V(0.0);
                     if (X.kind == 1) {
                         // rotated coefficients (src/translate.jl:555-826): m = 0, 1 of the rotated multipole and
                         // of the degree-k local (translate_multipole_to_local_z_m01_n!, :302-362)
-                        const V e0 = B::bperm(ME[0], c), e1 = B::bperm(MO[0], c);
-                        const V p0 = comp_of<0>(e0), p1r = comp_of<0>(e1), p1i = comp_of<1>(e1);
-                        eps_mp = (B::sqrt(p1r * p1r + p1i * p1i) + B::fabs(p0)) * np1_f * rmi_np2;
-                        if constexpr (LH) {
-                            const V c1r = comp_of<2>(e1), c1i = comp_of<3>(e1);
-                            eps_mp = eps_mp + B::sqrt(c1r * c1r + c1i * c1i) * np1_f * rmi_np2 * r_mp;
-                        }
+                        const V e0 = B::bperm(MEr[0], c), e1r = B::bperm(MOr[0], c), e1i = B::bperm(MOi[0], c);
+                        const V n1 = B::sqrt(e1r * e1r + e1i * e1i);
+                        eps_mp = phi_of(n1 + B::fabs(e0)) * np1_f * rmi_np2;
+                        if constexpr (LH) eps_mp = eps_mp + chi_of(n1) * np1_f * rmi_np2 * r_mp;
                         if (B::any(active && (eps_mp <= X.limit))) {
-                            const V l0 = B::bperm(L[LO<k>::v], c), l1 = B::bperm(L[LO<k>::v + ke], c);
-                            V q0 = comp_of<0>(l0), q1r = comp_of<0>(l1), q1i = comp_of<1>(l1);
+                            const V l0 = B::bperm(Lr[LO<k>::v], c), l1r = B::bperm(Lr[LO<k>::v + ke], c),
+                                    l1i = B::bperm(Li[LO<k>::v + ke], c);
+                            const V p0 = phi_of(l0);
+                            V p1r = phi_of(l1r), p1i = phi_of(l1i);
                             const double cl = rl_nm1 * nm1_f_inv;
                             if constexpr (LH) {
-                                const V d1r = comp_of<2>(l1), d1i = comp_of<3>(l1);
+                                const V d1r = chi_of(l1r), d1i = chi_of(l1i);
                                 const V ton = r * ik;
-                                q1r = q1r - ton * d1i;
-                                q1i = q1i + ton * d1r;
-                                eps_l = (B::fabs(q1r) + B::fabs(q1i) + B::fabs(q0)) * cl + B::sqrt(d1r * d1r + d1i * d1i) * (cl * X.r_l);
+                                p1r = p1r - ton * d1i;
+                                p1i = p1i + ton * d1r;
+                                eps_l = (B::fabs(p1r) + B::fabs(p1i) + B::fabs(p0)) * cl + B::sqrt(d1r * d1r + d1i * d1i) * (cl * X.r_l);
                             } else {
-                                eps_l = (B::fabs(q1r) + B::fabs(q1i) + B::fabs(q0)) * cl;
+                                eps_l = (B::fabs(p1r) + B::fabs(p1i) + B::fabs(p0)) * cl;
                             }
                         }
                     } else {
@@ -517,78 +531,89 @@ struct Engine {
                             eps_mp = eps_mp * rmi_np2 * r_mp;
                         }
                         if (B::any(active && (eps_mp <= X.limit))) {
-                            const V r_n = r * ik, r_np1 = r * ik1;
+                            const V qd = B::tod(q2);
+                            const V rk = B::sel(chi_lane, V(0.0), r * ik), rk1 = B::sel(chi_lane, r * ik1, V(0.0));
                             V lsum = V(0.0);
                             auto term = [&](auto par, auto RI) {
-                                constexpr int pr = decltype(par)::value, ri = decltype(RI)::value;
-                                constexpr int m0 = 8 * ri + pr;
-                                const I m = q * 2 + m0;
-                                const V x = pr ? L[LO<k>::v + ke + ri] : L[LO<k>::v + ri];
-                                V val = x;
+                                constexpr int pr = decltype(par)::value, ri = decltype(RI)::value, m0 = 8 * ri + pr;
+                                constexpr int at = LO<k>::v + (pr ? ke : 0) + ri;
+                                const I m = q2 + m0;
+                                V vr = Lr[at], vi = Li[at];
                                 if constexpr (LH) {
-                                    const V y = B::perm3(x);
-                                    const V rm = r_n * B::tod(m);
-                                    // chi of (k, m + 1): the odd register of the same lane for even m; for odd m
-                                    // the even part's next entry, one quad up (or register ri + 1 of quad 0)
-                                    V nxt;
+                                    // phi lanes: phi + i (r m / k) chi; chi lanes: chi_m - r / (k + 1) chi_(m + 1), the odd
+                                    // register of the same lane for even m; for odd m the even part's next entry, one quad up
+                                    // (or register ri + 1 of quad 0)
+                                    const V rm = rk * (qd + (double)m0);
+                                    V nr, ni;
                                     if constexpr (pr == 0) {
-                                        nxt = ri < ko ? L[LO<k>::v + ke + imin(ri, ko1 - 1)] : V(0.0);
+                                        nr = ri < ko ? Lr[LO<k>::v + ke + imin(ri, ko1 - 1)] : V(0.0);
+                                        ni = ri < ko ? Li[LO<k>::v + ke + imin(ri, ko1 - 1)] : V(0.0);
                                     } else {
-                                        const V hi = ri + 1 < ke ? L[LO<k>::v + imin(ri + 1, ke - 1)] : V(0.0);
-                                        const V tmp = B::sel(q == 0, hi, L[LO<k>::v + ri]);
-                                        nxt = B::bperm(tmp, ((q + 1) & 3) * 16 + c);
+                                        const V hr = ri + 1 < ke ? Lr[LO<k>::v + imin(ri + 1, ke - 1)] : V(0.0);
+                                        const V hi = ri + 1 < ke ? Li[LO<k>::v + imin(ri + 1, ke - 1)] : V(0.0);
+                                        const I up = ((q + 1) & 3) * 16 + c;
+                                        nr = B::bperm(B::sel(q == 0, hr, Lr[LO<k>::v + ri]), up);
+                                        ni = B::bperm(B::sel(q == 0, hi, Li[LO<k>::v + ri]), up);
                                     }
-                                    if constexpr (m0 + 7 > k) nxt = B::sel(m + 1 <= k, nxt, V(0.0));
-                                    val = B::sel(comp == 0, x - y * rm, B::sel(comp == 1, x + y * rm, x - nxt * r_np1));
+                                    if constexpr (m0 + 7 > k) {
+                                        const M has = m + 1 <= k;
+                                        nr = B::sel(has, nr, V(0.0));
+                                        ni = B::sel(has, ni, V(0.0));
+                                    }
+                                    const V yr = B::perm1(vr), yi = B::perm1(vi);
+                                    vr = B::fma(-rk1, nr, B::fma(-rm, yi, vr));
+                                    vi = B::fma(-rk1, ni, B::fma(rm, yr, vi));
                                 }
-                                const V t2 = val * val;
+                                const V t2 = B::fma(vr, vr, vi * vi);
                                 if constexpr (m0 + 6 <= k) {
                                     const V nt = B::lds(T.Lt, m + mnh(k - 1));
-                                    lsum = lsum + (t2 + B::perm1(t2)) * nt * nt;
+                                    lsum = B::fma(t2 * nt, nt, lsum);
                                 } else {
                                     const M ok = m <= k;
-                                    const V nt = B::lds(T.Lt, B::mini(m, k) + mnh(k - 1));
-                                    lsum = lsum + B::sel(ok, (t2 + B::perm1(t2)) * nt * nt, V(0.0));
+                                    const V nt = B::sel(ok, B::lds(T.Lt, B::mini(m, k) + mnh(k - 1)), V(0.0));
+                                    lsum = B::fma(t2 * nt, nt, lsum);
                                 }
                             };
                             sfor<0, ke>([&](auto EE) { term(std::integral_constant<int, 0>(), EE); });
                             sfor<0, ko>([&](auto OO) { term(std::integral_constant<int, 1>(), OO); });
-                            const V tl = B::quadsum(lsum);
-                            V lp, lc = V(0.0);
-                            if constexpr (LH) {
-                                const V o = B::perm2(tl);
-                                lp = B::sqrt(B::sel(pot == 0, tl, o));
-                                lc = B::sqrt(B::sel(pot == 1, tl, o));
-                            } else {
-                                lp = B::sqrt(tl);
-                            }
+                            const V tl = B::sqrt(B::quadsum(lsum));
                             const double cl = SQ3 * rl_nm1 * nm1_f_inv * iN;
-                            eps_l = lp * (X.kind == 3 ? cl : cl * X.r_l * ik);
-                            if (LH) eps_l = eps_l + lc * (cl * X.r_l);
+                            eps_l = phi_of(tl) * (X.kind == 3 ? cl : cl * X.r_l * ik);
+                            if constexpr (LH) eps_l = eps_l + chi_of(tl) * (cl * X.r_l);
                         }
                     }
                     pass = (eps_mp <= X.limit) && (eps_mp + eps_l * 2.0 <= X.limit);
                 }
+                const M newly = active && pass;
+                Pl = B::seli(newly, I(k - 1 + X.BE), Pl);
+                succ = succ || newly;
+                const M addk = active && (!pass || X.BE != 0);
+                active = active && !pass;
+                sfor<0, ke>([&](auto EE) {
+                    constexpr int e = decltype(EE)::value;
+                    MEr[e] = B::sel(addk, MEr[e], V(0.0));
+                    MEi[e] = B::sel(addk, MEi[e], V(0.0));
+                });
+                sfor<0, ko>([&](auto OO) {
+                    constexpr int o = decltype(OO)::value;
+                    MOr[o] = B::sel(addk, MOr[o], V(0.0));
+                    MOi[o] = B::sel(addk, MOi[o], V(0.0));
+                });
             }
-            const M newly = active && pass;
-            Pl = B::seli(newly, I(k - 1 + X.BE), Pl);
-            succ = succ || newly;
-            const M addk = active && (!pass || X.BE != 0);
-            active = active && !pass;
             // ---- M_k into the other degrees: L_j += F(j + k) M_k
-            sfor<0, ke>([&](auto EE) { ME[decltype(EE)::value] = B::sel(addk, ME[decltype(EE)::value], V(0.0)); });
-            sfor<0, ko>([&](auto OO) { MO[decltype(OO)::value] = B::sel(addk, MO[decltype(OO)::value], V(0.0)); });
             sfor<0, CAP + 1>([&](auto JJ) {
                 constexpr int j = decltype(JJ)::value;
                 if constexpr (j != k) {
                     const V fac = B::lds(W.F, fb + (k + j));
                     sfor<0, imin(KE(j), ke)>([&](auto EE) {
                         constexpr int e = decltype(EE)::value;
-                        L[LO<j>::v + e] = B::fma(fac, ME[e], L[LO<j>::v + e]);
+                        Lr[LO<j>::v + e] = B::fma(fac, MEr[e], Lr[LO<j>::v + e]);
+                        Li[LO<j>::v + e] = B::fma(fac, MEi[e], Li[LO<j>::v + e]);
                     });
                     sfor<0, imin(KO(j), ko)>([&](auto OO) {
                         constexpr int o = decltype(OO)::value;
-                        L[LO<j>::v + KE(j) + o] = B::fma(fac, MO[o], L[LO<j>::v + KE(j) + o]);
+                        Lr[LO<j>::v + KE(j) + o] = B::fma(fac, MOr[o], Lr[LO<j>::v + KE(j) + o]);
+                        Li[LO<j>::v + KE(j) + o] = B::fma(fac, MOi[o], Li[LO<j>::v + KE(j) + o]);
                     });
                 }
             });
@@ -603,28 +628,34 @@ struct Engine {
 
         // ---- Lamb-Helmholtz transform of the translated locals (transform_lh_local!, src/translate.jl:98-142)
         if constexpr (LH) {
+            const V rphi = B::sel(chi_lane, V(0.0), r);
             sfor<0, CAP + 1>([&](auto NN) {
                 constexpr int n = decltype(NN)::value;
                 if (n > kdone) return;
                 constexpr int ke = KE(n), ko = KO(n);
                 const I q = B::opaque(q0);
-                // phi += (r m / n) (-/+) chi on the phi lanes; chi -= r / (n + 1) chi_(n+1) on the chi lanes below
-                // the interaction's order. Per-lane coefficients, zero where a term does not apply, so each
-                // register is two multiply-adds with the reference's rounding (x + 0 y = x).
-                const V r_np1 = r * (1.0 / (n + 1));
-                const V r_n = r * (1.0 / (n > 0 ? n : 1));
-                const V bco = B::sel(chi_lane && (Pl > n), -r_np1, V(0.0));
+                // phi += i (r m / n) chi on the phi lanes; chi -= r / (n + 1) chi_(n+1) on the chi lanes below
+                // the interaction's order. Per-lane coefficients, zero where a term does not apply (x + 0 y = x).
+                const V r_n = rphi * (1.0 / (n > 0 ? n : 1)), qd = B::tod(q * 2);
+                const V bco = B::sel(chi_lane && (Pl > n), r * (-1.0 / (n + 1)), V(0.0));
                 auto lh = [&](auto par, auto RI) {
                     constexpr int pr = decltype(par)::value, ri = decltype(RI)::value;
                     constexpr int at = LOFF(n) + (pr ? ke : 0) + ri;
                     constexpr int nn = imin(n + 1, CAP);
                     constexpr int at1 = LOFF(nn) + (pr ? KE(nn) : 0) + ri;
-                    const I m = q * 2 + (8 * ri + pr);
-                    const V x = L[at];
-                    V nv = x;
-                    if constexpr (n > 0) nv = x + (phi_sign * (r_n * B::tod(m))) * B::perm3(x);
-                    if constexpr (n < CAP) nv = nv + bco * L[at1];
-                    L[at] = nv;
+                    V xr = Lr[at], xi = Li[at];
+                    if constexpr (n > 0) {
+                        const V rm = r_n * (qd + (double)(8 * ri + pr));
+                        const V yr = B::perm1(xr), yi = B::perm1(xi);
+                        xr = B::fma(-rm, yi, xr);
+                        xi = B::fma(rm, yr, xi);
+                    }
+                    if constexpr (n < CAP) {
+                        xr = B::fma(bco, Lr[at1], xr);
+                        xi = B::fma(bco, Li[at1], xi);
+                    }
+                    Lr[at] = xr;
+                    Li[at] = xi;
                 };
                 sfor<0, ke>([&](auto EE) { lh(std::integral_constant<int, 0>(), EE); });
                 sfor<0, ko>([&](auto OO) { lh(std::integral_constant<int, 1>(), OO); });
@@ -637,43 +668,46 @@ struct Engine {
             if (n > kdone) return;
             B::sched_fence();
             constexpr int ke = KE(n), ko = KO(n), ke1 = imax(ke, 1), ko1 = imax(ko, 1);
-            const I c = B::opaque(c0), q = B::opaque(q0), s = c / NC, comp = c % NC;
-            const I sb2 = s * (NS * 2);
-            RotLane RL = RL0;
-            RL.c = c;
-            RL.q = q;
-            RL.s = s;
-            const M on = valid && (Pl >= n);
-            V uE[ke1], uO[ko1], oE[ke1], oO[ko1];
-            auto scale = [&](auto par, auto RI, V& u) {
-                constexpr int pr = decltype(par)::value, ri = decltype(RI)::value;
-                const I m = q * 2 + (8 * ri + pr);
-                const M ok = on && (m <= n);
-                const V g = B::lds(T.ein, B::seli(ok, m, I(0)) + mnh(n - 1));
-                u = B::sel(ok, g * L[LO<n>::v + (pr ? ke : 0) + ri], V(0.0));
+            const I c = B::opaque(c0) & 15, q = B::opaque(q0) & 3;
+            const I s = LH ? c >> 1 : c, pot = LH ? c & 1 : I(0);
+            const I sb2 = s * (NS * 2), q2 = q * 2;
+            const M on = Pl >= n;
+            V uEr[ke1], uEi[ke1], uOr[ko1], uOi[ko1], oEr[ke1], oEi[ke1], oOr[ko1], oOi[ko1];
+            auto scale = [&](auto par, auto RI, V& ur, V& ui) {
+                constexpr int pr = decltype(par)::value, ri = decltype(RI)::value, m0 = 8 * ri + pr;
+                constexpr int at = LO<n>::v + (pr ? ke : 0) + ri;
+                const I mi = (PAD || m0 + 6 <= n) ? q2 + m0 : B::mini(q2 + m0, n);
+                V g = B::lds(T.ein, mi + mnh(n - 1));
+                if (!PAD && m0 + 6 > n) g = B::sel(q2 + m0 <= n, g, V(0.0));
+                if (err) g = B::sel(on, g, V(0.0));
+                ur = g * Lr[at];
+                ui = g * Li[at];
+                if constexpr (m0 == 0) ur = ur * B::sel(q == 0, V(0.5), V(1.0));
             };
-            sfor<0, ke>([&](auto EE) { scale(std::integral_constant<int, 0>(), EE, uE[decltype(EE)::value]); });
-            sfor<0, ko>([&](auto OO) { scale(std::integral_constant<int, 1>(), OO, uO[decltype(OO)::value]); });
-            if constexpr (ko == 0) uO[0] = V(0.0);
-            rotate<n>(T, W, T.eoh, -1.0, RL, uE, uO, oE, oO);
-            auto store = [&](auto par, auto RI, const V& o) {
-                constexpr int pr = decltype(par)::value, ri = decltype(RI)::value;
-                const I m = q * 2 + (8 * ri + pr);
-                const M ok = m <= n;
-                const I ei = sb2 + B::mini(m, n) * 2;
+            sfor<0, ke>([&](auto EE) { scale(std::integral_constant<int, 0>(), EE, uEr[decltype(EE)::value], uEi[decltype(EE)::value]); });
+            sfor<0, ko>([&](auto OO) { scale(std::integral_constant<int, 1>(), OO, uOr[decltype(OO)::value], uOi[decltype(OO)::value]); });
+            if constexpr (ko == 0) { uOr[0] = V(0.0); uOi[0] = V(0.0); }
+            rotate<n>(T, W, T.eoh, -1.0, c, q, s, uEr, uEi, uOr, uOi, oEr, oEi, oOr, oOi);
+            auto store = [&](auto par, auto RI, const V& xr, const V& xi) {
+                constexpr int m0 = 8 * decltype(RI)::value + decltype(par)::value;
+                const I m = q2 + m0;
+                const I ei = sb2 + ((PAD || m0 + 6 <= n) ? m : B::mini(m, n)) * 2;
                 const V er = B::lds(W.eim, ei), eimg = B::lds(W.eim, ei + 1);
-                const V y = o * er - (RL.nj * B::perm1(o)) * eimg;   // back_rotate_z! (src/rotate.jl:584-616)
-                const V z = B::template slotsum<NC>(y);
-                const M w = ok && (s == 0);
-                B::lds_add(W.acc, B::seli(w, (m + mnh(n - 1)) * NC + comp, I(0)), z, w);
+                // back_rotate_z! (src/rotate.jl:584-616)
+                const V zr = B::template slotsum<NP>(B::fma(xr, er, xi * eimg));
+                const V zi = B::template slotsum<NP>(B::fma(xi, er, -(xr * eimg)));
+                const M w = (c < NP) && (m0 + 6 <= n ? M(true) : (m <= n));
+                const I at = B::seli(w, m * NC + pot * 2, I(0)) + mnh(n - 1) * NC;
+                B::lds_add(W.acc, at, zr, w);
+                B::lds_add(W.acc, at + 1, zi, w);
             };
-            sfor<0, ke>([&](auto EE) { store(std::integral_constant<int, 0>(), EE, oE[decltype(EE)::value]); });
-            sfor<0, ko>([&](auto OO) { store(std::integral_constant<int, 1>(), OO, oO[decltype(OO)::value]); });
+            sfor<0, ke>([&](auto EE) { store(std::integral_constant<int, 0>(), EE, oEr[decltype(EE)::value], oEi[decltype(EE)::value]); });
+            sfor<0, ko>([&](auto OO) { store(std::integral_constant<int, 1>(), OO, oOr[decltype(OO)::value], oOi[decltype(OO)::value]); });
         });
         B::wsync();
 
         // ---- orders and flags
-        const M wr = valid && (q == 0) && (comp == 0);
+        const M wr = valid && (q0 == 0) && (pot0 == 0);
         B::sti(Bt.orders, B::seli(wr, li, I(0)), Pl, wr);
         const int mx = B::maxi(Pl, valid);
         if (mx > pmax) pmax = mx;

@@ -14,12 +14,13 @@ namespace fmmhip {
 // ================================ M2L on matrix cores, register-resident (m2l_mx.hpp)
 // Backend of the engine in m2l_mx.hpp for one gfx950 wavefront: a per-lane value is a register,
 // neighbouring lanes are read with DPP (quad permutations, row rotations), other lanes with
-// ds_bpermute (__shfl), and the product is v_mfma_f64_16x16x4f64.
+// ds_bpermute (__shfl), and the product is v_mfma_f64_4x4x4_4b_f64.
 template <int CTRL>
 __device__ __forceinline__ double dpp_d(double x) {
     const long long u = __double_as_longlong(x);
-    const int lo = __builtin_amdgcn_update_dpp((int)u, (int)u, CTRL, 0xF, 0xF, false);
-    const int hi = __builtin_amdgcn_update_dpp((int)(u >> 32), (int)(u >> 32), CTRL, 0xF, 0xF, false);
+    // every lane has a source: no old value to keep (with one, each move is preceded by a copy)
+    const int lo = __builtin_amdgcn_mov_dpp((int)u, CTRL, 0xF, 0xF, true);
+    const int hi = __builtin_amdgcn_mov_dpp((int)(u >> 32), CTRL, 0xF, 0xF, true);
     return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
 }
 static constexpr int DPP_QUAD(int a, int b, int c, int d) { return a | (b << 2) | (c << 4) | (d << 6); }
@@ -29,8 +30,8 @@ struct MxGpu {
     using V = double;
     using I = int;
     using M = bool;
-    typedef double V4 __attribute__((ext_vector_type(4)));
     using PV = const double*;
+    struct padded;   // the pi/2 tables are held in the zero-padded form
     static __device__ __forceinline__ I lane() { return (int)(threadIdx.x & 63); }
     static __device__ __forceinline__ V sel(M m, V a, V b) { return m ? a : b; }
     static __device__ __forceinline__ I seli(M m, I a, I b) { return m ? a : b; }
@@ -45,8 +46,6 @@ struct MxGpu {
     static __device__ __forceinline__ V fma(V a, V b, V c) { return ::fma(a, b, c); }
     static __device__ __forceinline__ V tod(I a) { return (double)a; }
     static __device__ __forceinline__ V perm1(V a) { return dpp_d<DPP_QUAD(1, 0, 3, 2)>(a); }
-    static __device__ __forceinline__ V perm2(V a) { return dpp_d<DPP_QUAD(2, 3, 0, 1)>(a); }
-    static __device__ __forceinline__ V perm3(V a) { return dpp_d<DPP_QUAD(3, 2, 1, 0)>(a); }
     static __device__ __forceinline__ V bperm(V a, I src) { return __shfl(a, src, 64); }
     static __device__ __forceinline__ V quadsum(V a) {
         const V b = a + __shfl_xor(a, 16, 64);
@@ -56,18 +55,16 @@ struct MxGpu {
     static __device__ __forceinline__ V slotsum(V a) {   // sum over lanes of the row with the same lane % NC
         V b = a + dpp_d<DPP_ROW_ROR(8)>(a);
         b = b + dpp_d<DPP_ROW_ROR(4)>(b);
-        if constexpr (NC == 2) b = b + dpp_d<DPP_ROW_ROR(2)>(b);
+        b = b + dpp_d<DPP_ROW_ROR(2)>(b);
+        if constexpr (NC == 1) b = b + dpp_d<DPP_ROW_ROR(1)>(b);
         return b;
     }
     template <int NC, int j>
-    static __device__ __forceinline__ V qbcast(V a) {
-        if constexpr (NC == 4) return dpp_d<DPP_QUAD(j, j, j, j)>(a);
-        else return dpp_d<DPP_QUAD(j, j, 2 + j, 2 + j)>(a);
+    static __device__ __forceinline__ V qbcast(V a) {   // of columns NC i + (0 .. NC - 1), the value of column NC i + j
+        static_assert(NC == 2, "columns come in pairs");
+        return dpp_d<DPP_QUAD(j, j, 2 + j, 2 + j)>(a);
     }
-    static __device__ __forceinline__ V4 zero4() { return V4{0.0, 0.0, 0.0, 0.0}; }
-    static __device__ __forceinline__ V get4(const V4& a, int r) { return a[r]; }
-    static __device__ __forceinline__ void set4(V4& a, int r, V x) { a[r] = x; }
-    static __device__ __forceinline__ void mfma(V a, V b, V4& d) { d = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, d, 0, 0, 0); }
+    static __device__ __forceinline__ V mfma4(V a, V b, V d) { return __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, d, 0, 0, 0); }
     static __device__ __forceinline__ bool any(M m) { return __ballot(m) != 0ull; }
     static __device__ __forceinline__ bool all(M m) { return __ballot(!m) == 0ull; }
     static __device__ __forceinline__ int maxi(I a, M m) {
@@ -107,11 +104,11 @@ struct MxGpu {
 
 template <int CAP, bool LH>
 __host__ __device__ constexpr int mx_wave_doubles() {
-    return (LH ? 4 : 2) * nh(CAP) + 4 * (LH ? 4 : 8) * (CAP + 1) + (LH ? 4 : 8) * (2 * CAP + 1);
+    return (LH ? 4 : 2) * nh(CAP) + 4 * (LH ? 8 : 16) * (CAP + 1) + (LH ? 8 : 16) * (2 * CAP + 1);
 }
 template <int CAP>
 __host__ __device__ constexpr int mx_shared_doubles() {
-    return mx::ALEN(CAP) + 6 * nh(CAP) + 4 * (CAP + 1);
+    return mx::PLEN(CAP) + 6 * nh(CAP) + 4 * (CAP + 1);
 }
 template <int CAP, bool LH>
 static size_t mx_lds_bytes(int nw) {
@@ -129,7 +126,7 @@ static size_t mx_lds_bytes(int nw) {
 // expansion (7.4 KB at cap 20) is written and read once per S interactions, 0.3 ms of the 1M ring's 30 ms.
 template <int CAP, bool LH>
 constexpr int mx_chunk() {
-    return (CAP <= 12 ? 2 : 4) * (LH ? 4 : 8);
+    return (CAP <= 12 ? 1 : 2) * (LH ? 8 : 16);
 }
 __host__ __device__ inline int64_t mx_first_slot(int64_t l0, int64_t box, int S) { return l0 / S + box; }
 
@@ -147,30 +144,44 @@ __device__ inline int mx_box_of(const int64_t* __restrict__ m2l_offsets, int n_b
     return __builtin_amdgcn_readfirstlane(lo);
 }
 
-// Persistent: every workgroup copies the tables into LDS once, then each wavefront takes chunks from a counter
-// (flags[2]) and runs their interactions BP at a time, summed in the wavefront's LDS.
-template <int CAP, bool LH, int NW, bool FULL>
-__global__ __launch_bounds__(64 * NW) void k_m2l_mx(const int32_t* __restrict__ m2l_targets,
+// Persistent: every workgroup copies the tables into LDS once, then each wavefront takes chunks, `grab` slots at a time,
+// from a counter (flags[2]) and runs their interactions BP at a time, summed in the wavefront's LDS.
+//
+// What bounds it: at cap 8 and 12 two or three wavefronts per SIMD, 40 % of the cycles on the vector ALU and matrix
+// cores, the rest waits on LDS and the gathered expansions (4M Plummer sphere, order 8, 22.9M interactions: 31.9 -> 9.0 ms,
+// 2.5e9 translations/s). At cap 16 and 20 the local expansion fills the registers (204 and 300 per lane; beyond 256
+// they move through accumulation registers), one wavefront per SIMD, LDS latency exposed (300k sphere, order 16:
+// 7.6 -> 3.7 ms, 6.3 ms when forced to two wavefronts; 1M ring, orders to 20: 28 -> 20.3 ms).
+template <int CAP, bool LH, int NW, bool ERR>
+__global__ __launch_bounds__(64 * NW, CAP <= 12 ? 2 : 1) void k_m2l_mx(const int32_t* __restrict__ m2l_targets,
                                                     const int64_t* __restrict__ m2l_offsets,
                                                     const int32_t* __restrict__ m2l_s, const Branch* __restrict__ tbr,
                                                     const Branch* __restrict__ sbr, const double* __restrict__ sex,
                                                     double* __restrict__ tex, double* __restrict__ part, int n_boxes,
-                                                    int64_t n_slots, int P, int PE, ErrParams E,
+                                                    int64_t n_slots, int grab, int P, int PE, ErrParams E,
                                                     const int32_t* __restrict__ perm, int32_t* __restrict__ orders,
                                                     int32_t* __restrict__ flags, int32_t* __restrict__ box_ok,
                                                     TablePtrs tb) {
-    using Eng = mx::Engine<MxGpu, CAP, LH, FULL>;
+    using Eng = mx::Engine<MxGpu, CAP, LH, ERR ? 1 : 0>;
     constexpr int H = nh(CAP), NC = Eng::NC, BP = Eng::BP, NS = CAP + 1;
     extern __shared__ double lds[];
     double* A = lds;
-    double* zin = A + mx::ALEN(CAP);
+    double* zin = A + mx::PLEN(CAP);
     double* zoh = zin + H;
     double* ein = zoh + H;
     double* eoh = ein + H;
     double* Mt = eoh + H;
     double* Lt = Mt + H;
     double* tf = Lt + H;
-    for (int i = threadIdx.x; i < mx::ALEN(CAP); i += blockDim.x) A[i] = tb.Ad[i];
+    for (int n = 0, at = 0; n <= CAP; ++n) {
+        const int ke = mx::KE(n), nb = ke + mx::KO(n);
+        for (int t = threadIdx.x; t < 16 * nb * nb; t += blockDim.x) {
+            const int rq = t / (16 * nb), kq = (t >> 4) % nb, i = (t >> 2) & 3, q = t & 3;
+            const int row = (rq < ke ? 8 * rq : 8 * (rq - ke) + 1) + 2 * i, col = (kq < ke ? 8 * kq : 8 * (kq - ke) + 1) + 2 * q;
+            A[at + t] = row <= n && col <= n ? tb.Ad[mx::ABASE(n) + row * mx::AST(n) + col] : 0.0;
+        }
+        at += 16 * nb * nb;
+    }
     for (int i = threadIdx.x; i < H; i += blockDim.x) {
         int n, m;
         idx_nm(i, n, m);
@@ -196,14 +207,25 @@ __global__ __launch_bounds__(64 * NW) void k_m2l_mx(const int32_t* __restrict__ 
     const int lane = lane_id();
     int pmax = 0, okf = 1;
     constexpr int S = mx_chunk<CAP, LH>();
+    int slot = 0, left = 0, box = 0;
+    int64_t lb = 0, le = 0;
     for (;;) {
-        int slot = 0;
-        if (lane == 0) slot = atomicAdd(flags + 2, 1);
-        slot = __builtin_amdgcn_readfirstlane(slot);
-        if (slot >= n_slots) break;
-        const int box = mx_box_of(m2l_offsets, n_boxes, slot, S, lane);
-        const int64_t lb = m2l_offsets[box], le = m2l_offsets[box + 1];
+        if (left == 0) {
+            if (lane == 0) slot = atomicAdd(flags + 2, grab);
+            slot = __builtin_amdgcn_readfirstlane(slot);
+            if (slot >= n_slots) break;
+            left = (int)min((int64_t)grab, n_slots - slot);
+            box = mx_box_of(m2l_offsets, n_boxes, slot, S, lane);
+            lb = m2l_offsets[box];
+            le = m2l_offsets[box + 1];
+        } else if (box + 1 < n_boxes && mx_first_slot(le, box + 1, S) <= slot) {
+            ++box;
+            lb = le;
+            le = m2l_offsets[box + 1];
+        }
         const int64_t l0 = lb + (slot - mx_first_slot(lb, box, S)) * S, l1 = min(le, l0 + S);
+        const int at = slot++;
+        --left;
         if (l0 >= le) continue;   // the box has one chunk fewer than slots
         for (int i = lane; i < NC * H; i += 64) W.acc[i] = 0.0;
         wave_sync();
@@ -234,7 +256,7 @@ __global__ __launch_bounds__(64 * NW) void k_m2l_mx(const int32_t* __restrict__ 
             double* dst = tex + (int64_t)it * HE4;
             for (int i = lane; i < NC * nh(P); i += 64) dst[4 * (i / NC) + i % NC] += W.acc[i];
         } else {
-            double* dst = part + (int64_t)slot * (NC * nh(P));
+            double* dst = part + (int64_t)at * (NC * nh(P));
             for (int i = lane; i < NC * nh(P); i += 64) dst[i] = W.acc[i];
         }
         wave_sync();
@@ -265,10 +287,10 @@ __global__ __launch_bounds__(256) void k_m2l_mx_sum(const int32_t* __restrict__ 
     }
 }
 
-template <int CAP, bool LH, int NW, bool FULL>
+template <int CAP, bool LH, int NW, bool ERR>
 static void launch_m2l_mx(Context& C, int p, int pe, const Lists& Ls, const Tree& st, Tree& tt_dst, const ErrParams& E,
                           const int32_t* perm, int32_t* flags, const TablePtrs& tb) {
-    auto kfn = k_m2l_mx<CAP, LH, NW, FULL>;
+    auto kfn = k_m2l_mx<CAP, LH, NW, ERR>;
     const size_t sh = mx_lds_bytes<CAP, LH>(NW);
     HIP_CHECK(hipFuncSetAttribute((const void*)kfn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sh));
     int per_cu = 0;
@@ -277,11 +299,16 @@ static void launch_m2l_mx(Context& C, int p, int pe, const Lists& Ls, const Tree
     // one slot past the last box's first for each of its chunks (its list may end inside a chunk)
     const int64_t slots = mx_first_slot(Ls.n_m2l, Ls.n_m2l_targets, mx_chunk<CAP, LH>());
     const int64_t want = (slots + NW - 1) / NW;
-    C.m2l_part.resize((size_t)slots * ((LH ? 4 : 2) * nh(p)));
     const unsigned grid = (unsigned)std::max<int64_t>(1, std::min<int64_t>(want, (int64_t)std::max(per_cu, 1) * C.n_cu));
+    // The counter is one address for all 8 XCDs and takes an increment about every 14 ns. Up to cap 12 a slot is less work
+    // than that over 2048-3072 wavefronts (4M Plummer sphere, order 8: 18.3 ms with one increment per slot, 9.0 ms with
+    // this rule), so a wavefront takes several at a time and still at least 16 times; above, a slot is ten times as long
+    // (1M ring, order cap 20: 20.3 ms with one, 21.8 ms with several).
+    const int grab = CAP <= 12 ? (int)std::max<int64_t>(1, std::min<int64_t>(16, slots / ((int64_t)16 * grid * NW))) : 1;
+    C.m2l_part.resize((size_t)slots * ((LH ? 4 : 2) * nh(p)));
     kfn<<<grid, 64 * NW, sh, C.stream>>>(Ls.m2l_targets.data(), Ls.m2l_offsets.data(), Ls.m2l_s.data(), tt_dst.branches.data(),
                                          st.branches.data(), st.expansions.data(), tt_dst.expansions.data(), C.m2l_part.data(),
-                                         (int)Ls.n_m2l_targets, slots, p, pe, E, perm, Ls.m2l_order.data(), flags,
+                                         (int)Ls.n_m2l_targets, slots, grab, p, pe, E, perm, Ls.m2l_order.data(), flags,
                                          Ls.track_box_ok ? const_cast<int32_t*>(Ls.m2l_box_ok.data()) : nullptr, tb);
     LAUNCH_CHECK();
     k_m2l_mx_sum<CAP, LH><<<(unsigned)Ls.n_m2l_targets, 256, 0, C.stream>>>(Ls.m2l_targets.data(), Ls.m2l_offsets.data(),
@@ -290,19 +317,22 @@ static void launch_m2l_mx(Context& C, int p, int pe, const Lists& Ls, const Tree
 }
 
 
-static constexpr int MX_NW = 4;   // wavefronts per workgroup (one per SIMD at the register use of the engine)
+static constexpr int MX_NW = 4;   // wavefronts per workgroup
 
-// the launch at order p <= CAP (CAP the smallest instantiated cap >= p)
+// the launch at order p <= CAP (CAP the smallest instantiated cap >= p). Fixed orders and error-controlled ones have an
+// engine each, so that the first holds none of the tests' values (order cap 8: 4,075 instructions and 166 registers
+// against 6,595 and 208 with the tests). Degree loops of fixed length (order equal to the cap) were dropped: without
+// the branch between degrees the scheduler mixes them and spills.
 template <int CAP>
 void run_m2l_mx_cap(Context& C, int p, bool LH, const Lists& Ls, const Tree& st, Tree& tt_dst, const ErrParams& E,
                     const int32_t* perm, int32_t* flags, const TablePtrs& tb) {
-    if (p == CAP) {   // degree loops of fixed length (34.1 against 34.4 ms on the 1M ring at cap 20)
-        if (LH) launch_m2l_mx<CAP, true, MX_NW, true>(C, p, p, Ls, st, tt_dst, E, perm, flags, tb);
-        else launch_m2l_mx<CAP, false, MX_NW, true>(C, p, p, Ls, st, tt_dst, E, perm, flags, tb);
-    } else {
-        if (LH) launch_m2l_mx<CAP, true, MX_NW, false>(C, p, p, Ls, st, tt_dst, E, perm, flags, tb);
-        else launch_m2l_mx<CAP, false, MX_NW, false>(C, p, p, Ls, st, tt_dst, E, perm, flags, tb);
-    }
+    auto run = [&](auto lh) {
+        constexpr bool L = decltype(lh)::value;
+        if (E.kind != 0) launch_m2l_mx<CAP, L, MX_NW, true>(C, p, p, Ls, st, tt_dst, E, perm, flags, tb);
+        else launch_m2l_mx<CAP, L, MX_NW, false>(C, p, p, Ls, st, tt_dst, E, perm, flags, tb);
+    };
+    if (LH) run(std::true_type());
+    else run(std::false_type());
 }
 
 }  // namespace fmmhip

@@ -9,7 +9,7 @@ import pytest
 import fastmultipole_amd as F
 from fastmultipole_amd import _lib, workloads as W
 
-CHUNK = {8: 2, 12: 2, 16: 4, 20: 4}   # batches per chunk at each order cap; a batch is 4 (vortex) or 8 interactions
+CHUNK = {8: 8, 12: 8, 16: 16, 20: 16}   # vortex interactions per chunk at each order cap; twice as many of one potential
 
 
 @pytest.mark.parametrize("S", [8, 16, 32])
@@ -27,7 +27,7 @@ def test_slots_of_boxes_never_overlap(S):
 @pytest.mark.parametrize("p", [7, 8, 12, 15, 20])
 def test_chunked_lists_match_the_wavefront_engine(p, kernel, monkeypatch):
     rows = W.plummer_sources(2600, seed=11) if kernel == _lib.POINT_SOURCE else W.uniform_vortices(2600, seed=11)
-    S = CHUNK[min(c for c in CHUNK if c >= p)] * (4 if kernel == _lib.POINT_VORTEX else 8)
+    S = CHUNK[min(c for c in CHUNK if c >= p)] * (1 if kernel == _lib.POINT_VORTEX else 2)
     outs = {}
     for engine in ("mx", "wave"):
         monkeypatch.setenv("FMMHIP_M2L_KERNEL", engine)
