@@ -131,6 +131,7 @@ struct Context {
     DBuf<double> l2p_coef;      // per-leaf local-to-body coefficients of the last L2P pass
     DBuf<double> m2m_slot;      // per-child translated multipoles of one level of the upward pass
     DBuf<unsigned long long> p2p_queue;   // work counter of the persistent nearfield launch
+    DBuf<double> panel_rec;     // frame and edge geometry of the nearfield's panels
     DBuf<double> direct_part;   // chunk sums of the split direct! form
     int n_cu = 0;               // compute units of the device (0 until first needed)
     DBuf<unsigned char> temp;   // scratch for sorts/scans

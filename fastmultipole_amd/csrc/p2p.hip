@@ -841,17 +841,34 @@ void run_direct_all(Context& C, int kernel, int64_t nt, const double* t_xyz, int
 namespace fmmhip {
 
 
+// every panel's frame and edge geometry, once per evaluation: a panel is read by about 60 target leaves, and forming it
+// in each one's tile took longer than that tile's pairs (one wavefront of four, 64 panels at a time)
+template <int NV, int NSTR>
+__global__ __launch_bounds__(P2P_BLOCK) void k_panel_records(const double* __restrict__ sx, const double* __restrict__ sy,
+                                                             const double* __restrict__ sz, const double* __restrict__ rows,
+                                                             int64_t ns, PanelStage<NV>* __restrict__ rec) {
+    const int64_t j = blockIdx.x * (int64_t)P2P_BLOCK + threadIdx.x;
+    if (j >= ns) return;
+    PanelStage<NV> P = {};
+    stage_panel<NV, NSTR>(sx, sy, sz, rows, ns, j, P);
+    rec[j] = P;
+}
+
+// One workgroup per target leaf. Bound by the pair's FP64 operations, about 700 issue slots: 54k source quadrilaterals,
+// potential and gradient, 1.62e8 pairs in 4.55 ms = 3.6e10 pairs/s (the reference's form, panels staged per tile: 12.1 ms).
+// At three wavefronts per SIMD instead of two the registers spill (5.0 ms). The next tile's panel indices are searched
+// while the current tile is copied.
 template <int NV, int MODE, bool PS, bool GS, bool HS>
 __global__ __launch_bounds__(P2P_BLOCK) void k_p2p_panel(const int32_t* __restrict__ dir_targets,
                                                          const int64_t* __restrict__ dir_offsets,
                                                          const int32_t* __restrict__ dir_s, const int64_t* __restrict__ dir_cum,
                                                          const Branch* __restrict__ tbr, const Branch* __restrict__ sbr,
                                                          const double* __restrict__ tx, const double* __restrict__ ty,
-                                                         const double* __restrict__ tz, const double* __restrict__ sx,
-                                                         const double* __restrict__ sy, const double* __restrict__ sz,
-                                                         const double* __restrict__ rows, int64_t ns, double* __restrict__ tout,
-                                                         int64_t nt, int64_t blk0) {
+                                                         const double* __restrict__ tz, const PanelStage<NV>* __restrict__ rec,
+                                                         double* __restrict__ tout, int64_t nt, int64_t blk0) {
+    constexpr int REC = sizeof(PanelStage<NV>) / sizeof(double);
     __shared__ PanelStage<NV> tile[PANEL_TILE];
+    __shared__ int64_t index[2][PANEL_TILE];
     const int64_t bi = blk0 + blockIdx.x;   // target leaf of this workgroup
     const Branch T = tbr[dir_targets[bi]];
     const int64_t l0 = dir_offsets[bi], l1 = dir_offsets[bi + 1];
@@ -867,11 +884,17 @@ __global__ __launch_bounds__(P2P_BLOCK) void k_p2p_panel(const int32_t* __restri
         double a[13];
 #pragma unroll
         for (int k = 0; k < 13; ++k) a[k] = 0.0;
-        for (int64_t f0 = base; f0 < end; f0 += PANEL_TILE) {
-            const int64_t cnt = std::min<int64_t>(PANEL_TILE, end - f0);
-            __syncthreads();
-            if (tid < cnt)
-                stage_panel<NV, MODE == 2 ? 2 : 1>(sx, sy, sz, rows, ns, stream_body(dir_s, dir_cum, sbr, l0, l1, f0 + tid), tile[tid]);
+        __syncthreads();   // the previous pass is done with the tile
+        if (tid < PANEL_TILE && base + tid < end) index[0][tid] = stream_body(dir_s, dir_cum, sbr, l0, l1, base + tid);
+        int cur = 0;
+        for (int64_t f0 = base; f0 < end; f0 += PANEL_TILE, cur ^= 1) {
+            const int cnt = (int)std::min<int64_t>(PANEL_TILE, end - f0);
+            __syncthreads();   // the previous tile's pairs are done, this tile's indices are written
+            const int64_t nf = f0 + PANEL_TILE + tid;
+            if (tid < PANEL_TILE && nf < end) index[cur ^ 1][tid] = stream_body(dir_s, dir_cum, sbr, l0, l1, nf);
+            double* dst = reinterpret_cast<double*>(tile);
+            for (int i = tid; i < cnt * REC; i += P2P_BLOCK)
+                dst[i] = reinterpret_cast<const double*>(rec + index[cur][i / REC])[i % REC];
             __syncthreads();
             if (active)
                 for (int s = lane_k; s < cnt; s += tpt) panel_pair_kind<NV, MODE, PS, GS, HS>(tile[s], xt, yt, zt, a);
@@ -895,7 +918,13 @@ static void launch_p2p_panel(Context& C, const Tree& tt, const Tree& st, const L
     const int64_t* cum = sv.dir_cum ? sv.dir_cum : L.dir_cum.data();
 #define PANEL_ARGS                                                                                                       \
     L.dir_targets.data(), L.dir_offsets.data(), L.dir_s.data(), cum, tt.branches.data(), sbr,                            \
-        tt.x.data(), tt.y.data(), tt.z.data(), st.x.data(), st.y.data(), st.z.data(), st.strength.data(), st.n, tout, nt, b0
+        tt.x.data(), tt.y.data(), tt.z.data(), rec, tout, nt, b0
+    // a tuple's panels are ranges of the concatenated bodies: records of all of them, those of other systems unread
+    C.panel_rec.resize((size_t)std::max<int64_t>(1, st.n) * (sizeof(PanelStage<NV>) / sizeof(double)));
+    PanelStage<NV>* rec = reinterpret_cast<PanelStage<NV>*>(C.panel_rec.data());
+    k_panel_records<NV, MODE == 2 ? 2 : 1><<<(unsigned)((st.n + P2P_BLOCK - 1) / P2P_BLOCK), P2P_BLOCK, 0, C.stream>>>(
+        st.x.data(), st.y.data(), st.z.data(), st.strength.data(), st.n, rec);
+    LAUNCH_CHECK();
     const int code = (PS ? 4 : 0) | (GS ? 2 : 0) | (HS ? 1 : 0);
     switch (code) {
         case 0: break;

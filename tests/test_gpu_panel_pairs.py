@@ -1,0 +1,82 @@
+"""The panel nearfield's closed form at targets where its terms degenerate: centroids (on the panel, on a quadrilateral's
+diagonal), edge midpoints and vertices of other panels, points a hair off a panel's plane, far points. direct! of
+every panel on every such target, to 1e-10 of the largest value of a quantity: what the solid angle
+enters (source panels' potential and gradient, dipole panels' potential) against the edge sums of Wilton et al. (1984) in
+extended precision, the rest against the oracle's reference form. (At triangles of size 1e-7 the reference's arctangents at
+a centroid, moved off the plane by eps(), are 1.9e-10 off.)"""
+import numpy as np
+import pytest
+
+import fastmultipole_amd as F
+from fastmultipole_amd import _lib, workloads as W
+from oracle import oracle as O
+
+KINDS = {"source-quads": (_lib.PANEL_SOURCE_QUAD, 6), "source-triangles": (_lib.PANEL_SOURCE_TRI, 4),
+         "dipole-quads": (_lib.PANEL_DIPOLE_QUAD, 7), "dipole-triangles": (_lib.PANEL_DIPOLE_TRI, 5)}
+
+
+def edge_sums(t, v, c):
+    """Potential and gradient slots of unit source panels v (n, nv, 3) with reference points c at t, and the potential slot of
+    unit dipole panels, summed, in long double."""
+    t, v, c = (np.asarray(x, dtype=np.longdouble) for x in (t, v, c))
+    e = v[:, 2] - v[:, 0]
+    ez = np.cross(v[:, 1] - v[:, 0], e)
+    ez /= np.sqrt((ez ** 2).sum(1))[:, None]
+    z = ((t[:, None] - c[None]) * ez[None]).sum(2)
+    z = np.where(z == 0, np.longdouble(2.0) ** -52, z)   # on the panel: its outer side
+    az = abs(z)
+    phi, beta, g = 0, 0, 0
+    for k in range(v.shape[1]):
+        a, b = v[:, k], v[:, (k + 1) % v.shape[1]]
+        length = np.sqrt(((b - a) ** 2).sum(1))
+        along = (b - a) / length[:, None]
+        out = np.cross(along, ez)
+        d = a[None] - t[:, None]
+        l0, p = (d * along[None]).sum(2), (d * out[None]).sum(2)
+        l1, h = l0 + length, p * p + z * z
+        r0, r1 = np.sqrt(h + l0 * l0), np.sqrt(h + l1 * l1)
+        f = np.log1p(2 * length / (r0 + r1 - length))
+        beta = beta + np.arctan2(p * l1, h + az * r1) - np.arctan2(p * l0, h + az * r0)
+        phi, g = phi + p * f, g + out[None] * f[..., None]
+    g = g + ez[None] * (np.sign(z) * beta)[..., None]
+    f4 = 1 / (4 * np.longdouble(np.pi))
+    return [(x.sum(1) * f4).astype(float) for x in (phi - az * beta, g, np.sign(z) * beta)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("scale", [1.0, 1e-6, 1e5])
+@pytest.mark.parametrize("name", list(KINDS))
+def test_direct_at_degenerate_targets(name, scale):
+    kernel, okind = KINDS[name]
+    rows, _ = W.sphere_panels(3, quads="quads" in name, seed=9)
+    rows[:, 4] = 1.0
+    if "quads" in name:   # squares in one plane: symmetric panels, whose edge angles at the centroid are right angles
+        sq = np.array([[[i, j, 3.0], [i + 1, j, 3.0], [i + 1, j + 1, 3.0], [i, j + 1, 3.0]] for i in range(2) for j in range(2)])
+        rows = np.concatenate([rows, W.panel_rows(sq, np.ones(4))])
+    v = rows[:, 5:].reshape(len(rows), -1, 3)
+    rng = np.random.default_rng(1)
+    n = v[:, 1] - v[:, 0]
+    n = np.cross(n, v[:, 2] - v[:, 0])
+    n /= np.linalg.norm(n, axis=1)[:, None]
+    off = np.exp(rng.uniform(np.log(1e-7), np.log(1.0), len(v)))[:, None]
+    t = np.concatenate([rows[:, :3], rows[:, :3] + off * n, rows[:, :3] - off * n,
+                        0.5 * (v[:, 0] + v[:, 1]) + 1e-3 * n, v[:, 2] - 1e-3 * n, 20.0 * rng.normal(size=(8, 3))])
+    rows = rows.copy()
+    rows[:, :4] *= scale
+    rows[:, 5:] *= scale
+    t = np.ascontiguousarray(t * scale)
+    out = np.zeros((len(t), 16))
+    ctx = F.default_context()
+    rows = np.ascontiguousarray(rows)
+    hess = "dipole" not in name   # a dipole panel's Hessian is not defined on its own plane
+    ctx.check(ctx.lib.fmmhip_direct(ctx._h, kernel, len(t), t.ctypes.data, len(rows), rows.ctypes.data, 1, 1, int(hess),
+                                    _lib.FP64, out.ctypes.data, 0))
+    ref = O.direct(okind, t, rows, True, True, hess)
+    phi, grad, dipole = edge_sums(t, rows[:, 5:].reshape(len(rows), -1, 3), rows[:, :3])
+    if "source" in name:
+        ref[:, 3], ref[:, 4:7] = phi, grad
+    else:
+        ref[:, 3] = dipole
+    for lo, hi in ((3, 4), (4, 7)) + (((7, 16),) if hess else ()):
+        assert np.isfinite(out[:, lo:hi]).all()
+        assert np.abs(out[:, lo:hi] - ref[:, lo:hi]).max() <= 1e-10 * np.abs(ref[:, lo:hi]).max(), (lo, hi)
