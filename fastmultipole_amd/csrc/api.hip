@@ -199,28 +199,40 @@ static void check_options(const fmmhip_options* o) {
     if (o->precision != FMMHIP_FP64 && o->precision != FMMHIP_MIXED) throw Error(FMMHIP_EINVAL, "unknown precision");
 }
 
+// Device time of a phase. The end is recorded with mark() and read with ms() once the evaluation has ended, so timing a
+// phase never makes the host wait for it: with a wait per phase (and the M2L's flags read as soon as it ended) the device
+// idled about 10 us at each of ten phases (1,000 vortices 1.60 -> 1.52 ms). Events are kept by the context and used again.
 struct Timer {
     Context& C;
-    hipEvent_t a, b;
+    hipEvent_t a = nullptr, b = nullptr;
     explicit Timer(Context& c) : C(c) {
-        HIP_CHECK(hipEventCreate(&a));
-        HIP_CHECK(hipEventCreate(&b));
+        a = take();
+        b = take();
         HIP_CHECK(hipEventRecord(a, C.stream));
     }
-    bool marked = false;
-    // records the end without waiting for it (read later by stop)
-    void mark() {
-        HIP_CHECK(hipEventRecord(b, C.stream));
-        marked = true;
+    Timer(const Timer&) = delete;
+    Timer& operator=(const Timer&) = delete;
+    ~Timer() {
+        C.timer_events.push_back(a);
+        C.timer_events.push_back(b);
     }
-    double stop() {
-        if (!marked) HIP_CHECK(hipEventRecord(b, C.stream));
+    void mark() { HIP_CHECK(hipEventRecord(b, C.stream)); }
+    double ms() {   // waits for the end
         HIP_CHECK(hipEventSynchronize(b));
-        float ms = 0;
-        HIP_CHECK(hipEventElapsedTime(&ms, a, b));
-        HIP_CHECK(hipEventDestroy(a));
-        HIP_CHECK(hipEventDestroy(b));
-        return ms;
+        float v = 0;
+        HIP_CHECK(hipEventElapsedTime(&v, a, b));
+        return v;
+    }
+private:
+    hipEvent_t take() {
+        if (C.timer_events.empty()) {
+            hipEvent_t e;
+            HIP_CHECK(hipEventCreate(&e));
+            return e;
+        }
+        hipEvent_t e = C.timer_events.back();
+        C.timer_events.pop_back();
+        return e;
     }
 };
 
@@ -282,6 +294,8 @@ static void release_context(Context& c) {
     c.tables = nullptr;
     c.tree_scratch = nullptr;
     c.list_scratch = nullptr;
+    for (hipEvent_t e : c.timer_events) (void)hipEventDestroy(e);
+    c.timer_events.clear();
     if (c.pinned) (void)hipHostFree(c.pinned);
     c.pinned = nullptr;
     if (c.stream) (void)hipStreamDestroy(c.stream);
@@ -397,14 +411,14 @@ static void eval_core(Eval& E, const fmmhip_options& o, fmmhip_stats* stats, boo
     const bool LH = has_vector_potential(E.kernel);
     const bool PS = o.scalar_potential != 0, GS = o.gradient != 0, HS = o.hessian != 0;
     Timer total(C);
-    double t_est = 0, t_gather = 0;
+    std::unique_ptr<Timer> tp, tu, te, tm, tl, td, tg;   // P2P, upward, estimate, M2L, L2L, L2P, gather
+    Context* far = nullptr;   // the context whose M2L flags are still to be read
     E.tout.resize((size_t)13 * std::max<int64_t>(1, E.nt));
     HIP_CHECK(hipMemsetAsync(E.tout.data(), 0, E.tout.size() * sizeof(double), C.stream));
     if (E.tt.n_branches) HIP_CHECK(hipMemsetAsync(E.tt.expansions.data(), 0, E.tt.expansions.size() * sizeof(double), C.stream));
     if (E.st.n_branches) HIP_CHECK(hipMemsetAsync(E.st.expansions.data(), 0, E.st.expansions.size() * sizeof(double), C.stream));
     E.pmax = 0;
     E.error_success = 1;
-    double t_p2p = 0, t_up = 0, t_m2l = 0, t_down = 0;
     if (E.nt > 0 && E.ns > 0) {
         // The nearfield (P2P) runs on the evaluation's stream while the far field
         // (estimate_influence, upward pass, M2L, L2L) runs on a second stream; L2P adds
@@ -420,14 +434,14 @@ static void eval_core(Eval& E, const fmmhip_options& o, fmmhip_stats* stats, boo
             stream_wait(F, C);
         }
         const bool estimate = !is_estimate && o.error_kind != FMMHIP_ERR_NONE && o.error_relative;
-        Timer tp(C);
+        tp.reset(new Timer(C));
         // Beside the far-field stream the nearfield leaves one workgroup slot per CU free: its
         // rate is about the same at 3 and 4 workgroups per CU, and the far field's kernels (the
         // estimate's tree, list and sort launches) are placed at once instead of waiting for
         // the nearfield's last workgroups.
         const int slots = &F != &C ? -C.p2p_free_slots : 0;
         eval_p2p(C, E, PS, GS, HS, o.precision, slots);
-        tp.mark();
+        tp->mark();
         // With estimate_influence on the far-field stream, the upward pass follows the nearfield on its
         // stream: it needs nothing of the estimate, so it runs beside the estimate's evaluation once the
         // nearfield is done (103.0 against 104.9 ms per evaluation of the 1M ring with it on the far-field
@@ -435,7 +449,6 @@ static void eval_core(Eval& E, const fmmhip_options& o, fmmhip_stats* stats, boo
         // nothing; 102.3 against 100.9 ms with it before the nearfield, beside the estimate's trees).
         // Without the estimate it stays on the far-field stream, beside the nearfield.
         const bool up_on_c = estimate && &F != &C;
-        std::unique_ptr<Timer> tu;
         if (up_on_c) {
             tu.reset(new Timer(C));
             eval_p2m(C, E, p);
@@ -447,22 +460,21 @@ static void eval_core(Eval& E, const fmmhip_options& o, fmmhip_stats* stats, boo
             // Measured alternatives: its trees and lists first, alone on the device (110.1 against 107.5 ms
             // per evaluation of the 1M ring: its evaluation then waits for the nearfield), and the upward
             // pass on a third stream beside it (109.0 ms: both then share the one free slot per CU).
-            Timer t(F);
+            te.reset(new Timer(F));
             estimate_build(E, o, F);
             estimate_eval(E, o, F);
-            t_est = t.stop();
+            te->mark();
         }
         if (!up_on_c) {
-            Timer t(F);
+            tu.reset(new Timer(F));
             eval_p2m(F, E, p);
             run_m2m(F, E.st, p, LH);
-            t_up = t.stop();
+            tu->mark();
         } else {
             stream_wait(F, C);
         }
         {
-            Timer t(F);
-            int32_t pmax = 0, ok = 1;
+            tm.reset(new Timer(F));
             const bool batch = !is_estimate && !E.seg.empty();
             E.lists.track_box_ok = batch;
             if (batch) {
@@ -472,8 +484,9 @@ static void eval_core(Eval& E, const fmmhip_options& o, fmmhip_stats* stats, boo
                 LAUNCH_CHECK();
             }
             run_m2l(F, E.tt, E.st, E.tt, E.lists, p, LH, o.error_kind, o.error_relative != 0, o.error_tolerance,
-                    o.error_bonus != 0, o.precision, batch ? nullptr : &pmax, &ok);
+                    o.error_bonus != 0, o.precision, nullptr, nullptr);
             if (batch) {
+                int32_t pmax = 0, ok = 1;
                 if (E.lists.n_m2l_targets > 0) {
                     k_system_status<<<grid_for(E.lists.n_m2l_targets, 256), 256, 0, F.stream>>>(
                         E.lists.m2l_targets.data(), E.lists.m2l_offsets.data(), E.lists.n_m2l_targets, E.lists.m2l_order.data(),
@@ -494,35 +507,42 @@ static void eval_core(Eval& E, const fmmhip_options& o, fmmhip_stats* stats, boo
                     pmax = std::max(pmax, h[2 * i]);
                     ok = ok && h[2 * i + 1];
                 }
+                E.pmax = pmax;
+                E.error_success = ok;
+                if (!ok) E.pmax += 1;
+            } else if (!is_estimate) {   // read once the evaluation has ended
+                HIP_CHECK(hipMemcpyAsync((char*)pinned_scratch(F) + 32, F.m2l_flags.data(), 2 * sizeof(int32_t),
+                                         hipMemcpyDeviceToHost, F.stream));
+                far = &F;
             }
-            E.pmax = pmax;
-            E.error_success = ok;
-            if (!ok) E.pmax += 1;
-            t_m2l = t.stop();
+            tm->mark();
         }
-        {
-            Timer t(F);
-            run_l2l(F, E.tt, p, LH);
-            t_down = t.stop();
-        }
-        if (tu) t_up = tu->stop();
+        tl.reset(new Timer(F));
+        run_l2l(F, E.tt, p, LH);
+        tl->mark();
         if (&F != &C) stream_wait(C, F);
-        {
-            Timer t(C);
-            run_l2p(C, E.tt, E.tout.data(), E.nt, p, LH, PS, GS, HS);
-            t_down += t.stop();
-        }
-        t_p2p = tp.stop();
+        td.reset(new Timer(C));
+        run_l2p(C, E.tt, E.tout.data(), E.nt, p, LH, PS, GS, HS);
+        td->mark();
     }
-    if (!is_estimate) {
-        Timer t(C);
-        E.tout_aos.resize((size_t)16 * std::max<int64_t>(1, E.nt));
-        gather_outputs(C, E.tt, E.tout.data(), E.tout_aos.data(), E.nt);
-        t_gather = t.stop();
+    if (is_estimate) {   // its results are used on this stream
+        E.ran = true;
+        return;
     }
-    const double t_tot = total.stop();
+    tg.reset(new Timer(C));
+    E.tout_aos.resize((size_t)16 * std::max<int64_t>(1, E.nt));
+    gather_outputs(C, E.tt, E.tout.data(), E.tout_aos.data(), E.nt);
+    tg->mark();
+    total.mark();
+    const double t_tot = total.ms();   // everything has ended: the far field joined this stream before the L2P
+    if (far) {
+        int32_t h[2];
+        std::memcpy(h, (const char*)far->pinned + 32, sizeof(h));
+        E.error_success = h[1];
+        E.pmax = h[0] + (h[1] ? 0 : 1);
+    }
     E.ran = true;
-    if (!is_estimate) E.keys_fresh = false;
+    E.keys_fresh = false;
     if (stats) {
         stats->pmax = E.pmax;
         stats->error_success = E.error_success;
@@ -531,13 +551,14 @@ static void eval_core(Eval& E, const fmmhip_options& o, fmmhip_stats* stats, boo
         stats->n_m2l = E.lists.n_m2l;
         stats->n_direct = E.lists.n_direct;
         stats->n_p2p_pairs = E.lists.n_pairs;
-        stats->ms_p2p = t_p2p;
-        stats->ms_upward = t_up;
-        stats->ms_m2l = t_m2l;
-        stats->ms_downward = t_down;
+        auto ms = [](const std::unique_ptr<Timer>& t) { return t ? t->ms() : 0.0; };
+        stats->ms_p2p = ms(tp);
+        stats->ms_upward = ms(tu);
+        stats->ms_m2l = ms(tm);
+        stats->ms_downward = ms(tl) + ms(td);
         stats->ms_total = t_tot;
-        stats->ms_estimate = t_est;
-        stats->ms_gather = t_gather;
+        stats->ms_estimate = ms(te);
+        stats->ms_gather = ms(tg);
     }
 }
 
@@ -825,23 +846,18 @@ fmmhip_status fmmhip_fmm(fmmhip_eval* ev, const fmmhip_options* o, fmmhip_stats*
     Context* C = ev->e.ctx;
     ABI_TRY(C, {
         check_options(o);
-        Timer t(*C);
-        double t_tree, t_lists;
-        {
-            Timer a(*C);
-            eval_build_trees(ev->e, *o);
-            t_tree = a.stop();
-        }
-        {
-            Timer a(*C);
-            eval_build_lists(ev->e, *o);
-            t_lists = a.stop();
-        }
+        Timer t(*C), t_tree(*C);
+        eval_build_trees(ev->e, *o);
+        t_tree.mark();
+        Timer t_lists(*C);
+        eval_build_lists(ev->e, *o);
+        t_lists.mark();
         eval_core(ev->e, *o, stats, false);
-        double tt = t.stop();
+        t.mark();
+        const double tt = t.ms();
         if (stats) {
-            stats->ms_tree = t_tree;
-            stats->ms_lists = t_lists;
+            stats->ms_tree = t_tree.ms();
+            stats->ms_lists = t_lists.ms();
             stats->ms_total = tt;
         }
     });

@@ -136,7 +136,8 @@ struct Context {
     int n_cu = 0;               // compute units of the device (0 until first needed)
     DBuf<unsigned char> temp;   // scratch for sorts/scans
     DBuf<unsigned char> sort_work;   // radix sort: digit counts, offsets, keys and values between passes
-    void* pinned = nullptr;     // 64 bytes of pinned host memory for scalar read-backs
+    void* pinned = nullptr;     // 64 bytes of pinned host memory for scalar read-backs (the M2L's flags at byte 32)
+    std::vector<hipEvent_t> timer_events;   // events of finished phase timers, for the next ones
     // Launch sequences without host synchronisation may be captured in graphs and replayed. Off for
     // contexts that share the device with other threads (the request server's workers): a
     // device-synchronising call there (hipFree) while a stream is being captured invalidates the capture.
