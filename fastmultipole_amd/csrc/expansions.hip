@@ -2275,8 +2275,13 @@ __global__ __launch_bounds__(64) void k_p2m(const Branch* __restrict__ br, const
 // x0+xv and calculate_ib! at x0 (:112-213), each degree from the previous one
 // (get_nm1 rules, :77-110), then M += |xu x xv| (-1)^(n+m) conj(i_n^m) * (-q)
 // (source) or the dipole conversion source_to_dipole! of i with moment -q n
-// (:251-278). One wavefront per leaf; lane m carries coefficient m of the
-// current degree for all three recurrences at once (one barrier per degree).
+// (:251-278). One wavefront per leaf. A group of P + 1 lanes takes a triangle, lane m
+// of it coefficient m of the current degree for all three recurrences at once (one
+// barrier per degree), and the 64 / (P + 1) groups take triangles side by side, each
+// summing into its own copy of the leaf's expansion; the copies are added in group
+// order. Bound by the chain of degrees, each with a few LDS and FP64 latencies: 20,184
+// quadrilaterals, order 6, 280 us with one triangle per wavefront at a time (7 of 64
+// lanes) and six divisions per degree, 37 us with nine and one.
 // Quadrilaterals are the triangles (v1, v2, v3) and (v1, v3, v4) with the unit
 // normal of each triangle.
 
@@ -2290,10 +2295,10 @@ __device__ inline void nm1_vals(const double* A, int n, int m, double q[6]) {
     if (m + 1 < n) { q[4] = A[2 * (b + m + 1)]; q[5] = A[2 * (b + m + 1) + 1]; } else { q[4] = 0.0; q[5] = 0.0; }
 }
 
+// valid: this lane's group has a triangle; m: the lane's rank in its group
 template <bool DIPOLE>
 __device__ void p2m_triangle(const double* v1, const double* v2, const double* v3, const double* center, double strength, int P,
-                             double* Q, double* J, double* I, double* Macc) {
-    const int m = (int)threadIdx.x;
+                             bool valid, int m, double* Q, double* J, double* I, double* Macc) {
     const double x0[3] = {v1[0] - center[0], v1[1] - center[1], v1[2] - center[2]};
     const double xu[3] = {v2[0] - v1[0], v2[1] - v1[1], v2[2] - v1[2]};
     const double xv[3] = {v3[0] - v1[0], v3[1] - v1[1], v3[2] - v1[2]};
@@ -2309,8 +2314,9 @@ __device__ void p2m_triangle(const double* v1, const double* v2, const double* v
         dqx = -c0 / area2 * strength; dqy = -c1 / area2 * strength; dqz = -c2 / area2 * strength;
     }
     const double w = DIPOLE ? area2 : area2 * (-strength);
+    double r0 = 1.0, r1 = 1.0, r2 = 0.5;   // 1 / n, 1 / (n + 1), 1 / (n + 2)
     for (int n = 0; n <= P; ++n) {
-        const bool act = m <= n;
+        const bool act = valid && m <= n;
         const int i = nh(n - 1) + m;
         double qr = 0.0, qi = 0.0, jr = 0.0, ji = 0.0, ir = 0.0, ii = 0.0, dr = 0.0, di = 0.0;
         if (act) {
@@ -2319,14 +2325,14 @@ __device__ void p2m_triangle(const double* v1, const double* v2, const double* v
             } else {
                 double a[6];
                 nm1_vals(Q, n, m, a);   // calculate_q! (:112-139)
-                qr = (-(qxr * a[1] + qxi * a[0]) - (qer * a[5] + qei * a[4]) - qz * a[2]) / (double)n;
-                qi = ((qxr * a[0] - qxi * a[1]) + (qer * a[4] - qei * a[5]) - qz * a[3]) / (double)n;
+                qr = (-(qxr * a[1] + qxi * a[0]) - (qer * a[5] + qei * a[4]) - qz * a[2]) * r0;
+                qi = ((qxr * a[0] - qxi * a[1]) + (qer * a[4] - qei * a[5]) - qz * a[3]) * r0;
                 nm1_vals(J, n, m, a);   // calculate_pj! (:146-176)
-                jr = (-(jxr * a[1] + jxi * a[0]) - (jer * a[5] + jei * a[4]) - jz * a[2] + qr) / (double)(n + 1);
-                ji = ((jxr * a[0] - jxi * a[1]) + (jer * a[4] - jei * a[5]) - jz * a[3] + qi) / (double)(n + 1);
+                jr = (-(jxr * a[1] + jxi * a[0]) - (jer * a[5] + jei * a[4]) - jz * a[2] + qr) * r1;
+                ji = ((jxr * a[0] - jxi * a[1]) + (jer * a[4] - jei * a[5]) - jz * a[3] + qi) * r1;
                 nm1_vals(I, n, m, a);   // calculate_ib! (:183-213)
-                ir = (-(ixr * a[1] + ixi * a[0]) - (ier * a[5] + iei * a[4]) - iz * a[2] + jr) / (double)(n + 2);
-                ii = ((ixr * a[0] - ixi * a[1]) + (ier * a[4] - iei * a[5]) - iz * a[3] + ji) / (double)(n + 2);
+                ir = (-(ixr * a[1] + ixi * a[0]) - (ier * a[5] + iei * a[4]) - iz * a[2] + jr) * r2;
+                ii = ((ixr * a[0] - ixi * a[1]) + (ier * a[4] - iei * a[5]) - iz * a[3] + ji) * r2;
                 if (DIPOLE) {   // source_to_dipole! (:251-278) from i of degree n-1
                     dr = -dqx * 0.5 * (a[5] + a[1]) + dqy * 0.5 * (a[4] - a[0]) - dqz * a[2];
                     di = dqx * 0.5 * (a[4] + a[0]) + dqy * 0.5 * (a[5] - a[1]) - dqz * a[3];
@@ -2343,6 +2349,9 @@ __device__ void p2m_triangle(const double* v1, const double* v2, const double* v
             I[2 * i] = ir; I[2 * i + 1] = ii;
         }
         __syncthreads();   // degree n published
+        r0 = r1;
+        r1 = r2;
+        r2 = 1.0 / (double)(n + 3);
     }
 }
 
@@ -2350,33 +2359,44 @@ template <int KERNEL>
 __global__ __launch_bounds__(64) void k_p2m_panel(const Branch* __restrict__ br, const int64_t* __restrict__ leaf_index,
                                                   const double* __restrict__ rows, int64_t ns, double* __restrict__ ex, int P,
                                                   int srow, int voff) {
-    extern __shared__ double lds[];
+    extern __shared__ double lds[];   // per group: Q, J, I and the group's expansion, 2 H doubles each
     constexpr int NV = panel_vertices(KERNEL);
     constexpr bool DIPOLE = panel_dipole(KERNEL);
-    const int H = nh(P);
-    double* Q = lds;
+    const int H = nh(P), G = 64 / (P + 1);
+    const int g = (int)threadIdx.x / (P + 1), m = (int)threadIdx.x % (P + 1);
+    double* Q = lds + (size_t)(g < G ? g : 0) * 8 * H;   // the lanes left over never write
     double* J = Q + 2 * H;
     double* I = J + 2 * H;
     double* Macc = I + 2 * H;
     const int64_t ib = leaf_index[blockIdx.x];
     const Branch B = br[ib];
-    for (int k = threadIdx.x; k < 2 * H; k += 64) Macc[k] = 0.0;
+    for (int k = threadIdx.x; k < G * 2 * H; k += 64) lds[(size_t)(k / (2 * H)) * 8 * H + 6 * H + k % (2 * H)] = 0.0;
     __syncthreads();
-    for (int64_t j = B.first; j < B.first + B.n_bodies; ++j) {
-        double v[NV][3];
+    const int64_t ntri = B.n_bodies * (NV - 2);
+    for (int64_t base = 0; base < ntri; base += G) {
+        const bool valid = g < G && base + g < ntri;
+        const int64_t tri = valid ? base + g : base;
+        const int64_t j = B.first + tri / (NV - 2);
+        const int t = (int)(tri % (NV - 2));
+        double v[3][3];
 #pragma unroll
-        for (int k = 0; k < NV; ++k)
-#pragma unroll
-            for (int a = 0; a < 3; ++a) v[k][a] = rows[(int64_t)(voff + 3 * k + a) * ns + j];
+        for (int a = 0; a < 3; ++a) {
+            v[0][a] = rows[(int64_t)(voff + a) * ns + j];
+            v[1][a] = rows[(int64_t)(voff + 3 * (t + 1) + a) * ns + j];
+            v[2][a] = rows[(int64_t)(voff + 3 * (t + 2) + a) * ns + j];
+        }
         const double q = rows[(int64_t)srow * ns + j];   // strength row srow, vertices from row voff
-#pragma unroll
-        for (int t = 0; t < NV - 2; ++t)
-            p2m_triangle<DIPOLE>(v[0], v[t + 1], v[t + 2], B.source_center, q, P, Q, J, I, Macc);
+        p2m_triangle<DIPOLE>(v[0], v[1], v[2], B.source_center, q, P, valid, m, Q, J, I, Macc);
     }
     __syncthreads();
     for (int k = threadIdx.x; k < H; k += 64) {
-        ex[ib * 4 * H + 4 * k] += Macc[2 * k];
-        ex[ib * 4 * H + 4 * k + 1] += Macc[2 * k + 1];
+        double re = 0.0, im = 0.0;
+        for (int h = 0; h < G; ++h) {
+            re += lds[(size_t)h * 8 * H + 6 * H + 2 * k];
+            im += lds[(size_t)h * 8 * H + 6 * H + 2 * k + 1];
+        }
+        ex[ib * 4 * H + 4 * k] += re;
+        ex[ib * 4 * H + 4 * k + 1] += im;
     }
 }
 
@@ -2386,7 +2406,7 @@ void run_p2m(Context& C, int kernel, Tree& st, int p, const Branch* sbr) {
     if (st.n_leaves == 0) return;
     TablePtrs tb = ptrs(C);
     if (is_panel(kernel)) {
-        const size_t sh = sizeof(double) * 8 * nh(p);
+        const size_t sh = sizeof(double) * 8 * nh(p) * (64 / (p + 1));   // at most 44 KB (order 20)
 #define FMMHIP_P2M_PANEL(K, SROW, VOFF)                                                                                \
     k_p2m_panel<K><<<(unsigned)st.n_leaves, 64, sh, C.stream>>>(sbr, st.leaf_index.data(), st.strength.data(),             \
                                                                st.n, st.expansions.data(), p, SROW, VOFF)
