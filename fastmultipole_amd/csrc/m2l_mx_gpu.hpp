@@ -211,10 +211,17 @@ __global__ __launch_bounds__(64 * NW, CAP <= 12 ? 2 : 1) void k_m2l_mx(const int
     int64_t lb = 0, le = 0;
     for (;;) {
         if (left == 0) {
-            if (lane == 0) slot = atomicAdd(flags + 2, grab);
-            slot = __builtin_amdgcn_readfirstlane(slot);
-            if (slot >= n_slots) break;
-            left = (int)min((int64_t)grab, n_slots - slot);
+            if (grab == 0) {   // one slot per wavefront
+                if (slot) break;
+                slot = (int)blockIdx.x * NW + __builtin_amdgcn_readfirstlane(wave_id());
+                if (slot >= n_slots) break;
+                left = 1;
+            } else {
+                if (lane == 0) slot = atomicAdd(flags + 2, grab);
+                slot = __builtin_amdgcn_readfirstlane(slot);
+                if (slot >= n_slots) break;
+                left = (int)min((int64_t)grab, n_slots - slot);
+            }
             box = mx_box_of(m2l_offsets, n_boxes, slot, S, lane);
             lb = m2l_offsets[box];
             le = m2l_offsets[box + 1];
@@ -302,9 +309,11 @@ static void launch_m2l_mx(Context& C, int p, int pe, const Lists& Ls, const Tree
     const unsigned grid = (unsigned)std::max<int64_t>(1, std::min<int64_t>(want, (int64_t)std::max(per_cu, 1) * C.n_cu));
     // The counter is one address for all 8 XCDs and takes an increment about every 14 ns. Up to cap 12 a slot is less work
     // than that over 2048-3072 wavefronts (4M Plummer sphere, order 8: 18.3 ms with one increment per slot, 9.0 ms with
-    // this rule), so a wavefront takes several at a time and still at least 16 times; above, a slot is ten times as long
-    // (1M ring, order cap 20: 20.3 ms with one, 21.8 ms with several).
-    const int grab = CAP <= 12 ? (int)std::max<int64_t>(1, std::min<int64_t>(16, slots / ((int64_t)16 * grid * NW))) : 1;
+    // several), so a wavefront takes two to sixteen at a time, a sixth of its share; above, a slot is ten times as long
+    // (1M ring, order cap 20: 20.3 ms with one, 21.8 ms with several). With a wavefront for every slot there is no counter
+    // (grab 0): a small launch otherwise spends a third of its time on it.
+    const int64_t waves = (int64_t)grid * NW, share = slots / waves;
+    const int grab = slots <= waves ? 0 : CAP <= 12 && share >= 4 ? (int)std::max<int64_t>(2, std::min<int64_t>(16, share / 6)) : 1;
     C.m2l_part.resize((size_t)slots * ((LH ? 4 : 2) * nh(p)));
     kfn<<<grid, 64 * NW, sh, C.stream>>>(Ls.m2l_targets.data(), Ls.m2l_offsets.data(), Ls.m2l_s.data(), tt_dst.branches.data(),
                                          st.branches.data(), st.expansions.data(), tt_dst.expansions.data(), C.m2l_part.data(),
