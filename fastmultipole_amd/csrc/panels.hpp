@@ -97,16 +97,17 @@ __device__ inline double panel_sqrt(double x) {
     return fma(fma(-r, r, x), 0.5 * y, r);
 }
 
-// log((rp - d) / (rp + d)), 0 <= d <= rp: 2 atanh(s) - e ln 2 with the ratio's power of two e split off so that
+// log((rp - d) / (rp + d)), d >= 0: 2 atanh(s) - e ln 2 with the ratio's power of two e split off so that
 // |s| <= 3 - 2 sqrt(2), then the series of atanh to s^21 (the next term is below 2^-56 of the sum). Without a power of
 // two s = -d / rp, so a far panel's small logarithm keeps its relative accuracy; a wavefront whose pairs are all far
-// (d <= 0.17 rp) skips the split.
+// (d <= 0.17 rp) skips the split. For a target on the edge rp - d rounds to zero or a few ulps below it (the distances and
+// the length are rounded apart): either takes the reference's eps() for zero, so the logarithm is large and bounded.
 __device__ inline double edge_log(double rp, double d) {
     const double EPS = 2.220446049250313e-16;   // the reference's eps() perturbation
     double a = -d, b = rp, shift = 0.0;
     if (__builtin_amdgcn_ballot_w64(d > 0.17 * rp)) {
         double num = rp - d;
-        if (num == 0.0) num = EPS;
+        if (num <= 0.0) num = EPS;
         const double den = rp + d;
         int e = __builtin_amdgcn_frexp_exp(den) - __builtin_amdgcn_frexp_exp(num);
         double m = __builtin_amdgcn_ldexp(num, e);

@@ -1,5 +1,6 @@
 """The panel nearfield's closed form at targets where its terms degenerate: centroids (on the panel, on a quadrilateral's
-diagonal), edge midpoints and vertices of other panels, points a hair off a panel's plane, far points. direct! of
+diagonal), points 1e-3 off edge midpoints and vertices, points a hair off a panel's plane, far points; and, in tests of
+their own, targets exactly on edges and at vertices. direct! of
 every panel on every such target, to 1e-10 of the largest value of a quantity: what the solid angle
 enters (source panels' potential and gradient, dipole panels' potential) against the edge sums of Wilton et al. (1984) in
 extended precision, the rest against the oracle's reference form. (At triangles of size 1e-7 the reference's arctangents at
@@ -35,7 +36,8 @@ def edge_sums(t, v, c):
         l0, p = (d * along[None]).sum(2), (d * out[None]).sum(2)
         l1, h = l0 + length, p * p + z * z
         r0, r1 = np.sqrt(h + l0 * l0), np.sqrt(h + l1 * l1)
-        f = np.log1p(2 * length / (r0 + r1 - length))
+        # on an edge the difference rounds to zero or below it: p f is then below any rounding of phi
+        f = np.log1p(2 * length / np.maximum(r0 + r1 - length, np.longdouble(2.0) ** -100))
         beta = beta + np.arctan2(p * l1, h + az * r1) - np.arctan2(p * l0, h + az * r0)
         phi, g = phi + p * f, g + out[None] * f[..., None]
     g = g + ez[None] * (np.sign(z) * beta)[..., None]
@@ -80,3 +82,45 @@ def test_direct_at_degenerate_targets(name, scale):
     for lo, hi in ((3, 4), (4, 7)) + (((7, 16),) if hess else ()):
         assert np.isfinite(out[:, lo:hi]).all()
         assert np.abs(out[:, lo:hi] - ref[:, lo:hi]).max() <= 1e-10 * np.abs(ref[:, lo:hi]).max(), (lo, hi)
+
+
+def direct(kernel, rows, t, hessian=False):
+    """direct! of every panel row on every target: potential, gradient (and Hessian) slots."""
+    rows, t = np.ascontiguousarray(rows), np.ascontiguousarray(t)
+    out = np.zeros((len(t), 16))
+    ctx = F.default_context()
+    ctx.check(ctx.lib.fmmhip_direct(ctx._h, kernel, len(t), t.ctypes.data, len(rows), rows.ctypes.data, 1, 1, int(hessian),
+                                    _lib.FP64, out.ctypes.data, 0))
+    return out
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("scale", [1.0, 1e-6, 1e5])
+@pytest.mark.parametrize("name", ["source-quads", "source-triangles", "source-dipole-quads", "source-dipole-triangles"])
+def test_targets_on_edges_and_at_vertices(name, scale):
+    """Targets exactly on panels' edges (midpoints, other fractions) and at their vertices, where the sum of the distances to
+    an edge's ends rounds to its length or below it. The potential is finite there: against the edge sums in extended
+    precision. The gradient is logarithmically infinite: each edge's logarithm is at most the one of the reference's eps()
+    perturbation, |log(eps() / 2d)| < 60 at these scales."""
+    rows, _ = W.sphere_panels(5, quads="quads" in name, seed=4)
+    rows[:, 4] = 1.0
+    v = rows[:, 5:].reshape(len(rows), -1, 3)
+    nv = v.shape[1]
+    rng = np.random.default_rng(2)
+    edge = rng.integers(0, nv, len(v))
+    a, b = v[np.arange(len(v)), edge], v[np.arange(len(v)), (edge + 1) % nv]
+    s = rng.uniform(0.0, 1.0, len(v))[:, None]
+    t = np.concatenate([0.5 * (a + b), a + s * (b - a), a]) * scale
+    rows = rows.copy()
+    rows[:, :4] *= scale
+    rows[:, 5:] *= scale
+    phi, _, _ = edge_sums(t, rows[:, 5:].reshape(len(rows), -1, 3), rows[:, :3])
+    if "dipole" in name:   # no dipole strength: the source's potential and gradient
+        kernel = _lib.PANEL_SOURCE_DIPOLE_QUAD if nv == 4 else _lib.PANEL_SOURCE_DIPOLE_TRI
+        out = direct(kernel, np.insert(rows, 5, 0.0, axis=1), t)
+    else:
+        out = direct(KINDS[name][0], rows, t)
+        assert np.isfinite(out[:, 4:7]).all()
+        assert np.abs(out[:, 4:7]).max() < len(v) * nv * 60 / (4 * np.pi)
+    assert np.isfinite(out[:, 3]).all()
+    assert np.abs(out[:, 3] - phi).max() <= 1e-10 * np.abs(phi).max()
