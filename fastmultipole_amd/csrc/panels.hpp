@@ -165,11 +165,15 @@ __device__ inline void panel_terms(const PanelStage<NV>& P, double tx, double ty
     // The solid angle: edge k adds atan(p l1 / (h + |z| r1)) - atan(p l0 / (h + |z| r0)), p the target's signed distance
     // from the edge's line in the plane, l0 and l1 the edge's ends along it, h = p^2 + z^2. An edge's angle lies in
     // (-pi, pi); two of one sign whose product's imaginary part has the other sign sum past pi. Lengths are taken in
-    // units of the first edge's power of two, so products of all edges stay in range.
+    // units of the power of two above the distance R to the farthest vertex: |p|, |l|, |z| <= R, so an edge's number is at
+    // most 8 and the product of all of them in range whatever the edges' lengths are.
     double angle = 0.0;
     if (ANGLE) {
         const double az = fabs(dz);
-        const int e0 = -2 * __builtin_amdgcn_frexp_exp(P.ds[0]);
+        int far = __double2hiint(rs[0]);   // distances are positive: their high words are in the order of the distances
+#pragma unroll
+        for (int k = 1; k < NV; ++k) far = max(far, __double2hiint(rs[k]));
+        const int e0 = 2 * (1022 - (far >> 20));
         double re = 0.0, im = 0.0;
         int turns = 0;
 #pragma unroll

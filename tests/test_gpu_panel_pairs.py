@@ -124,3 +124,28 @@ def test_targets_on_edges_and_at_vertices(name, scale):
         assert np.abs(out[:, 4:7]).max() < len(v) * nv * 60 / (4 * np.pi)
     assert np.isfinite(out[:, 3]).all()
     assert np.abs(out[:, 3] - phi).max() <= 1e-10 * np.abs(phi).max()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("distance", [1.0, 1e3, 3e4])
+@pytest.mark.parametrize("name", ["source-quads", "dipole-quads"])
+def test_sliver_edges_seen_from_afar(name, distance):
+    """Pole quadrilaterals of a sphere meshed in latitude and longitude: the first edge is sin(pi) = 1.2e-16 of the radius
+    wide, up to 1e21 times shorter than the distance. The solid angle's eight edge ends each carry a rounding of at most
+    8 2^-53 of a right angle's tangent, 32 2^-52 in all; the rest of a value is good to 1e-13."""
+    n, polar = 20, np.array([np.pi, np.pi - 0.1])
+    phi = np.linspace(0.0, 2 * np.pi, n + 1)
+    point = lambda th, ph: np.stack([np.sin(th) * np.cos(ph), np.sin(th) * np.sin(ph), np.cos(th) + 0 * ph], axis=-1)
+    lo, hi = point(polar[0], phi), point(polar[1], phi)
+    rows = W.panel_rows(np.stack([lo[:-1], lo[1:], hi[1:], hi[:-1]], axis=1), np.ones(n))
+    t = np.random.default_rng(6).normal(size=(40, 3))
+    t *= distance / np.linalg.norm(t, axis=1)[:, None]
+    out = direct(KINDS[name][0], rows, t)
+    ref, grad, dipole = edge_sums(t, rows[:, 5:].reshape(n, 4, 3), rows[:, :3])
+    angle = n * 32 * 2.0 ** -52 / (4 * np.pi)
+    assert np.isfinite(out[:, 3:7]).all()
+    if name == "dipole-quads":
+        assert np.abs(out[:, 3] - dipole).max() <= angle
+    else:
+        assert np.abs(out[:, 3] - ref).max() <= 1e-13 * np.abs(ref).max() + angle * 1.1 * distance
+        assert np.abs(out[:, 4:7] - grad).max() <= 1e-13 * np.abs(grad).max() + angle
