@@ -72,8 +72,8 @@ __device__ inline void stage_panel(const double* __restrict__ px, const double* 
         const double dx = vx[(k + 1) % NV] - vx[k], dy = vy[(k + 1) % NV] - vy[k];
         const double d = sqrt(dx * dx + dy * dy);
         P.ds[k] = d;
-        P.tx[k] = dx / d;
-        P.ty[k] = dy / d;
+        P.tx[k] = d == 0.0 ? 0.0 : dx / d;   // a vertex given twice: an edge that adds nothing
+        P.ty[k] = d == 0.0 ? 0.0 : dy / d;
     }
 }
 

@@ -149,3 +149,24 @@ def test_sliver_edges_seen_from_afar(name, distance):
     else:
         assert np.abs(out[:, 3] - ref).max() <= 1e-13 * np.abs(ref).max() + angle * 1.1 * distance
         assert np.abs(out[:, 4:7] - grad).max() <= 1e-13 * np.abs(grad).max() + angle
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("repeat", [[0, 1, 2, 2], [0, 1, 2, 0]], ids=["third-vertex-twice", "first-vertex-twice"])
+@pytest.mark.parametrize("name", ["source", "dipole", "source-dipole"])
+def test_quadrilaterals_with_a_repeated_vertex(name, repeat):
+    """Triangles handed over as quadrilaterals with a vertex given twice: the edge of no length adds nothing, so every output
+    is the triangle kernel's up to rounding (1e-12 of the largest value)."""
+    kinds = {"source": (_lib.PANEL_SOURCE_TRI, _lib.PANEL_SOURCE_QUAD), "dipole": (_lib.PANEL_DIPOLE_TRI, _lib.PANEL_DIPOLE_QUAD),
+             "source-dipole": (_lib.PANEL_SOURCE_DIPOLE_TRI, _lib.PANEL_SOURCE_DIPOLE_QUAD)}[name]
+    rows = W.sphere_source_dipole_panels(3, quads=False, seed=3)[0]
+    if "-" not in name:
+        rows = np.delete(rows, 5, axis=1)
+    at = rows.shape[1] - 9
+    v = rows[:, at:].reshape(-1, 3, 3)
+    quads = np.concatenate([rows[:, :at], v[:, repeat].reshape(len(v), 12)], axis=1)
+    rng = np.random.default_rng(8)
+    t = np.concatenate([rng.normal(size=(40, 3)), 0.2 * rng.normal(size=(10, 3))])
+    tri, quad = (direct(k, r, t, hessian=True) for k, r in zip(kinds, (rows, quads)))
+    for lo, hi in ((3, 4), (4, 7), (7, 16)):
+        assert np.abs(quad[:, lo:hi] - tri[:, lo:hi]).max() <= 1e-12 * np.abs(tri[:, lo:hi]).max(), (lo, hi)
