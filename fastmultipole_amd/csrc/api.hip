@@ -185,6 +185,8 @@ static void eval_p2p(Context& C, Eval& E, bool PS, bool GS, bool HS, int precisi
         SourceView sv;
         sv.branches = E.sys_branches.data() + s * nb;
         sv.dir_cum = E.sys_dir_cum.data() + s * (nd + 1);
+        sv.off = E.sys_off[s];
+        sv.n = E.sys_off[s + 1] - E.sys_off[s];
         run_p2p(C, E.sys_kind[s], E.tt, E.st, E.lists, E.tout.data(), E.nt, PS, GS, HS, precision, 0, -1, slots, sv);
     }
 }

@@ -258,10 +258,12 @@ void build_lists(Context& C, const Tree& tt, const Tree& st, Lists& L, int64_t l
 // kernels run as workgroups taking leaves from the context's queue: at most `slots` per CU
 // (0: as many as fit, < 0: that many fewer than fit).
 // One system of several sharing the source tree: its bodies' range in each leaf (a copy of the tree's
-// branches with the leaves' first / n_bodies replaced) and the direct list's prefix of its counts.
+// branches with the leaves' first / n_bodies replaced), the direct list's prefix of its counts, and its original
+// indices off .. off + n - 1.
 struct SourceView {
     const Branch* branches = nullptr;
     const int64_t* dir_cum = nullptr;
+    int64_t off = 0, n = 0;
 };
 void run_p2p(Context& C, int kernel, const Tree& tt, const Tree& st, const Lists& L, double* tout, int64_t nt,
              bool PS, bool GS, bool HS, int precision,

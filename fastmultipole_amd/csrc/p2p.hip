@@ -615,6 +615,7 @@ static void launch_p2p(Context& C, const Tree& tt, const Tree& st, const Lists& 
 #undef P2P_ARGS
 }
 
+void run_panel_records(Context& C, int kernel, const Tree& st, SourceView sv);
 void run_p2p_panels(Context& C, int kernel, const Tree& tt, const Tree& st, const Lists& L, double* tout, int64_t nt, bool PS,
                     bool GS, bool HS, int64_t b0, int64_t b1, SourceView sv);
 // targets b0 .. b1 - 1 of the direct list's CSR, none inside another
@@ -626,6 +627,7 @@ void run_direct_panels(Context& C, int kernel, int64_t nt, const double* t_xyz, 
 void run_p2p(Context& C, int kernel, const Tree& tt, const Tree& st, const Lists& L, double* tout, int64_t nt, bool PS, bool GS,
              bool HS, int precision, int64_t b0, int64_t b1, int slots, SourceView sv) {
     if (b1 < 0) b1 = L.n_direct_targets;
+    if (is_panel(kernel) && b0 < b1 && (PS || GS || HS)) run_panel_records(C, kernel, st, sv);
     if (!L.dir_level_split.empty()) {   // nested targets: one launch per level, ancestors first
         const std::vector<int64_t>& s = L.dir_level_split;
         for (size_t l = 0; l + 1 < s.size(); ++l) {
@@ -879,16 +881,19 @@ namespace fmmhip {
 
 
 // every panel's frame and edge geometry, once per evaluation: a panel is read by about 60 target leaves, and forming it
-// in each one's tile took longer than that tile's pairs (one wavefront of four, 64 panels at a time)
+// in each one's tile took longer than that tile's pairs (one wavefront of four, 64 panels at a time). A single system's
+// records are in the tree's order; one of a tuple's systems, whose panels lie apart in it, has its records in original
+// order (at: the tree's position of each original index), so that the other systems' bodies take no memory.
 template <int NV, int NSTR>
 __global__ __launch_bounds__(P2P_BLOCK) void k_panel_records(const double* __restrict__ sx, const double* __restrict__ sy,
                                                              const double* __restrict__ sz, const double* __restrict__ rows,
-                                                             int64_t ns, PanelStage<NV>* __restrict__ rec) {
-    const int64_t j = blockIdx.x * (int64_t)P2P_BLOCK + threadIdx.x;
-    if (j >= ns) return;
+                                                             int64_t ns, const int64_t* __restrict__ at, int64_t n,
+                                                             PanelStage<NV>* __restrict__ rec) {
+    const int64_t i = blockIdx.x * (int64_t)P2P_BLOCK + threadIdx.x;
+    if (i >= n) return;
     PanelStage<NV> P = {};
-    stage_panel<NV, NSTR>(sx, sy, sz, rows, ns, j, P);
-    rec[j] = P;
+    stage_panel<NV, NSTR>(sx, sy, sz, rows, ns, at ? at[i] : i, P);
+    rec[i] = P;
 }
 
 // One workgroup per target leaf. Bound by the pair's FP64 operations, about 700 issue slots: 54k source quadrilaterals,
@@ -902,6 +907,7 @@ __global__ __launch_bounds__(P2P_BLOCK) void k_p2p_panel(const int32_t* __restri
                                                          const Branch* __restrict__ tbr, const Branch* __restrict__ sbr,
                                                          const double* __restrict__ tx, const double* __restrict__ ty,
                                                          const double* __restrict__ tz, const PanelStage<NV>* __restrict__ rec,
+                                                         const int64_t* __restrict__ orig, int64_t off,
                                                          double* __restrict__ tout, int64_t nt, int64_t blk0) {
     constexpr int REC = sizeof(PanelStage<NV>) / sizeof(double);
     __shared__ PanelStage<NV> tile[PANEL_TILE];
@@ -913,6 +919,10 @@ __global__ __launch_bounds__(P2P_BLOCK) void k_p2p_panel(const int32_t* __restri
     const int tid = threadIdx.x;
     const LeafLanes LL = leaf_lanes(T.n_bodies);
     const int tpt = LL.t, lane_k = LL.lane_k;
+    auto record = [&](int64_t f) {   // of stream position f
+        const int64_t j = stream_body(dir_s, dir_cum, sbr, l0, l1, f);
+        return orig ? orig[j] - off : j;
+    };
     for (int64_t c0 = 0; c0 < T.n_bodies; c0 += LL.per_pass) {
         const int64_t ti = leaf_unit(LL, c0);
         const bool active = LL.gl < LL.gpw && ti < T.n_bodies;
@@ -922,13 +932,13 @@ __global__ __launch_bounds__(P2P_BLOCK) void k_p2p_panel(const int32_t* __restri
 #pragma unroll
         for (int k = 0; k < 13; ++k) a[k] = 0.0;
         __syncthreads();   // the previous pass is done with the tile
-        if (tid < PANEL_TILE && base + tid < end) index[0][tid] = stream_body(dir_s, dir_cum, sbr, l0, l1, base + tid);
+        if (tid < PANEL_TILE && base + tid < end) index[0][tid] = record(base + tid);
         int cur = 0;
         for (int64_t f0 = base; f0 < end; f0 += PANEL_TILE, cur ^= 1) {
             const int cnt = (int)std::min<int64_t>(PANEL_TILE, end - f0);
             __syncthreads();   // the previous tile's pairs are done, this tile's indices are written
             const int64_t nf = f0 + PANEL_TILE + tid;
-            if (tid < PANEL_TILE && nf < end) index[cur ^ 1][tid] = stream_body(dir_s, dir_cum, sbr, l0, l1, nf);
+            if (tid < PANEL_TILE && nf < end) index[cur ^ 1][tid] = record(nf);
             double* dst = reinterpret_cast<double*>(tile);
             for (int i = tid; i < cnt * REC; i += P2P_BLOCK)
                 dst[i] = reinterpret_cast<const double*>(rec + index[cur][i / REC])[i % REC];
@@ -946,6 +956,26 @@ __global__ __launch_bounds__(P2P_BLOCK) void k_p2p_panel(const int32_t* __restri
     }
 }
 
+template <int NV, int NSTR>
+static void launch_panel_records(Context& C, const Tree& st, SourceView sv) {
+    const int64_t n = sv.branches ? sv.n : st.n;
+    if (n <= 0) return;
+    C.panel_rec.resize((size_t)n * (sizeof(PanelStage<NV>) / sizeof(double)));
+    k_panel_records<NV, NSTR><<<(unsigned)((n + P2P_BLOCK - 1) / P2P_BLOCK), P2P_BLOCK, 0, C.stream>>>(
+        st.x.data(), st.y.data(), st.z.data(), st.strength.data(), st.n, sv.branches ? st.inverse_sort.data() + sv.off : nullptr, n,
+        reinterpret_cast<PanelStage<NV>*>(C.panel_rec.data()));
+    LAUNCH_CHECK();
+}
+
+void run_panel_records(Context& C, int kernel, const Tree& st, SourceView sv) {
+    switch (kernel) {
+        case FMMHIP_PANEL_SOURCE_TRI: case FMMHIP_PANEL_DIPOLE_TRI: launch_panel_records<3, 1>(C, st, sv); break;
+        case FMMHIP_PANEL_SOURCE_DIPOLE_TRI: launch_panel_records<3, 2>(C, st, sv); break;
+        case FMMHIP_PANEL_SOURCE_DIPOLE_QUAD: launch_panel_records<4, 2>(C, st, sv); break;
+        default: launch_panel_records<4, 1>(C, st, sv); break;
+    }
+}
+
 template <int NV, int MODE>
 static void launch_p2p_panel(Context& C, const Tree& tt, const Tree& st, const Lists& L, double* tout, int64_t nt, bool PS,
                              bool GS, bool HS, int64_t b0, int64_t b1, SourceView sv) {
@@ -953,15 +983,10 @@ static void launch_p2p_panel(Context& C, const Tree& tt, const Tree& st, const L
     if (nblk <= 0) return;
     const Branch* sbr = sv.branches ? sv.branches : st.branches.data();
     const int64_t* cum = sv.dir_cum ? sv.dir_cum : L.dir_cum.data();
+    const PanelStage<NV>* rec = reinterpret_cast<const PanelStage<NV>*>(C.panel_rec.data());
 #define PANEL_ARGS                                                                                                       \
     L.dir_targets.data(), L.dir_offsets.data(), L.dir_s.data(), cum, tt.branches.data(), sbr,                            \
-        tt.x.data(), tt.y.data(), tt.z.data(), rec, tout, nt, b0
-    // a tuple's panels are ranges of the concatenated bodies: records of all of them, those of other systems unread
-    C.panel_rec.resize((size_t)std::max<int64_t>(1, st.n) * (sizeof(PanelStage<NV>) / sizeof(double)));
-    PanelStage<NV>* rec = reinterpret_cast<PanelStage<NV>*>(C.panel_rec.data());
-    k_panel_records<NV, MODE == 2 ? 2 : 1><<<(unsigned)((st.n + P2P_BLOCK - 1) / P2P_BLOCK), P2P_BLOCK, 0, C.stream>>>(
-        st.x.data(), st.y.data(), st.z.data(), st.strength.data(), st.n, rec);
-    LAUNCH_CHECK();
+        tt.x.data(), tt.y.data(), tt.z.data(), rec, sv.branches ? st.sort_index.data() : nullptr, sv.off, tout, nt, b0
     const int code = (PS ? 4 : 0) | (GS ? 2 : 0) | (HS ? 1 : 0);
     switch (code) {
         case 0: break;

@@ -235,3 +235,26 @@ def test_tuple_rejects_bad_input():
     assert lib.fmmhip_eval_set_tuple_leaf_sizes(ev._h, 2, counts.ctypes.data) == 0
     assert lib.fmmhip_fgs_setup(ev._h, ctypes.byref(opt), _lib.INFLUENCE_POTENTIAL) == _lib.FMMHIP_EINVAL
     ev.close()
+
+
+def _free_bytes():
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert _lib.load().hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0   # the runtime the library is linked to
+    return free.value
+
+
+def test_panel_records_are_the_panel_system_s_alone():
+    """A few panels beside many particles: the nearfield's device memory is its lists and the panels' own records (280 bytes
+    each), not records of the particles (0.3 GB here)."""
+    _say("[gpu] tuple of 1M vortices and 96 panels")
+    rows = W.sphere_panels(4, seed=3)[0]
+    ev = F.Evaluation()
+    ev.set_tuple([_lib.POINT_VORTEX, _lib.PANEL_SOURCE_QUAD], [W.uniform_vortices(1000000, seed=2), rows])
+    opt = dict(expansion_order=4, leaf_size_source=200, multipole_acceptance=0.5)
+    ev.fmm(F.make_options(nearfield=False, self_induced=False, **opt))
+    before = _free_bytes()
+    ev.fmm(F.make_options(**opt))
+    grown = before - _free_bytes()
+    ev.close()
+    print(f"grown by {grown / 2**20:.0f} MiB", flush=True)
+    assert grown < 250 * 2**20
