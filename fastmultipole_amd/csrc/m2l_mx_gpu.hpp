@@ -130,6 +130,14 @@ constexpr int mx_chunk() {
 }
 __host__ __device__ inline int64_t mx_first_slot(int64_t l0, int64_t box, int S) { return l0 / S + box; }
 
+// Bytes of partial expansions at most. The slots of larger launches are taken in passes: the pass from w0 to w1 takes
+// every chunk of the boxes whose first slot lies in it, up to `span` slots past w1 (a list holds a source branch once, so
+// its chunks are no more than n_branches / S), and k_m2l_mx_sum adds them before the next pass. A box is summed whole in
+// one pass, so its sum does not depend on where the passes end. One pass for 4M bodies at order 8 (1.1 GB) or the 1M ring
+// at order 20 (1.0 GB); without a bound 2.5M uniform vortices at order 20 (37M interactions) took 20.7 GiB, and 428 ms
+// against 430 ms in ten passes.
+static constexpr int64_t MX_PART_BYTES = (int64_t)2 << 30;
+
 // the box whose slots hold slot w: the last one whose first slot is not above w (64 candidates per step)
 __device__ inline int mx_box_of(const int64_t* __restrict__ m2l_offsets, int n_boxes, int64_t w, int S, int lane) {
     int lo = 0, len = n_boxes;
@@ -145,7 +153,7 @@ __device__ inline int mx_box_of(const int64_t* __restrict__ m2l_offsets, int n_b
 }
 
 // Persistent: every workgroup copies the tables into LDS once, then each wavefront takes chunks, `grab` slots at a time,
-// from a counter (flags[2]) and runs their interactions BP at a time, summed in the wavefront's LDS.
+// from a counter (flags[2], from 0 in every pass) and runs their interactions BP at a time, summed in the wavefront's LDS.
 //
 // What bounds it: at cap 8 and 12 two or three wavefronts per SIMD, 40 % of the cycles on the vector ALU and matrix
 // cores, the rest waits on LDS and the gathered expansions (4M Plummer sphere, order 8, 22.9M interactions: 31.9 -> 9.0 ms,
@@ -158,7 +166,7 @@ __global__ __launch_bounds__(64 * NW, CAP <= 12 ? 2 : 1) void k_m2l_mx(const int
                                                     const int32_t* __restrict__ m2l_s, const Branch* __restrict__ tbr,
                                                     const Branch* __restrict__ sbr, const double* __restrict__ sex,
                                                     double* __restrict__ tex, double* __restrict__ part, int n_boxes,
-                                                    int64_t n_slots, int grab, int P, int PE, ErrParams E,
+                                                    int w0, int w1, int wend, int grab, int P, int PE, ErrParams E,
                                                     const int32_t* __restrict__ perm, int32_t* __restrict__ orders,
                                                     int32_t* __restrict__ flags, int32_t* __restrict__ box_ok,
                                                     TablePtrs tb) {
@@ -207,20 +215,20 @@ __global__ __launch_bounds__(64 * NW, CAP <= 12 ? 2 : 1) void k_m2l_mx(const int
     const int lane = lane_id();
     int pmax = 0, okf = 1;
     constexpr int S = mx_chunk<CAP, LH>();
-    int slot = 0, left = 0, box = 0;
+    int slot = -1, left = 0, box = 0;
     int64_t lb = 0, le = 0;
     for (;;) {
         if (left == 0) {
             if (grab == 0) {   // one slot per wavefront
-                if (slot) break;
-                slot = (int)blockIdx.x * NW + __builtin_amdgcn_readfirstlane(wave_id());
-                if (slot >= n_slots) break;
+                if (slot >= 0) break;
+                slot = w0 + (int)blockIdx.x * NW + __builtin_amdgcn_readfirstlane(wave_id());
+                if (slot >= wend) break;
                 left = 1;
             } else {
-                if (lane == 0) slot = atomicAdd(flags + 2, grab);
+                if (lane == 0) slot = w0 + atomicAdd(flags + 2, grab);
                 slot = __builtin_amdgcn_readfirstlane(slot);
-                if (slot >= n_slots) break;
-                left = (int)min((int64_t)grab, n_slots - slot);
+                if (slot >= wend) break;
+                left = min(grab, wend - slot);
             }
             box = mx_box_of(m2l_offsets, n_boxes, slot, S, lane);
             lb = m2l_offsets[box];
@@ -230,10 +238,11 @@ __global__ __launch_bounds__(64 * NW, CAP <= 12 ? 2 : 1) void k_m2l_mx(const int
             lb = le;
             le = m2l_offsets[box + 1];
         }
-        const int64_t l0 = lb + (slot - mx_first_slot(lb, box, S)) * S, l1 = min(le, l0 + S);
-        const int at = slot++;
+        const int first = (int)mx_first_slot(lb, box, S);
+        const int64_t l0 = lb + (int64_t)(slot - first) * S, l1 = min(le, l0 + S);
+        const int at = slot++ - w0;
         --left;
-        if (l0 >= le) continue;   // the box has one chunk fewer than slots
+        if (l0 >= le || first < w0 || first >= w1) continue;   // one chunk fewer than slots, or a box of another pass
         for (int i = lane; i < NC * H; i += 64) W.acc[i] = 0.0;
         wave_sync();
         const int32_t it = m2l_targets[box];
@@ -274,18 +283,21 @@ __global__ __launch_bounds__(64 * NW, CAP <= 12 ? 2 : 1) void k_m2l_mx(const int
     }
 }
 
-// adds the chunks of each box of more than one, in chunk order, to its target's expansion
+// adds the chunks of each of the pass's boxes of more than one, in chunk order, to its target's expansion, and sets the
+// counter back for the next pass
 template <int CAP, bool LH>
 __global__ __launch_bounds__(256) void k_m2l_mx_sum(const int32_t* __restrict__ m2l_targets,
                                                     const int64_t* __restrict__ m2l_offsets, double* __restrict__ tex,
-                                                    const double* __restrict__ part, int P, int PE) {
+                                                    const double* __restrict__ part, int w0, int w1, int P, int PE,
+                                                    int32_t* __restrict__ flags) {
     constexpr int S = mx_chunk<CAP, LH>(), NC = LH ? 4 : 2;
     const int box = blockIdx.x;
-    const int64_t l0 = m2l_offsets[box], l1 = m2l_offsets[box + 1];
-    if (l1 - l0 <= S) return;
+    if (box == 0 && threadIdx.x == 0) flags[2] = 0;
+    const int64_t l0 = m2l_offsets[box], l1 = m2l_offsets[box + 1], first = mx_first_slot(l0, box, S);
+    if (l1 - l0 <= S || first < w0 || first >= w1) return;
     const int64_t n = (l1 - l0 + S - 1) / S;
     const int len = NC * nh(P);
-    const double* src = part + mx_first_slot(l0, box, S) * len;
+    const double* src = part + (first - w0) * len;
     double* dst = tex + (int64_t)m2l_targets[box] * (4 * (int64_t)nh(PE));
     for (int i = threadIdx.x; i < len; i += 256) {
         double v = src[i];
@@ -303,26 +315,34 @@ static void launch_m2l_mx(Context& C, int p, int pe, const Lists& Ls, const Tree
     int per_cu = 0;
     HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(kfn), 64 * NW, sh));
     if (!C.n_cu) HIP_CHECK(hipDeviceGetAttribute(&C.n_cu, hipDeviceAttributeMultiprocessorCount, C.device));
+    constexpr int S = mx_chunk<CAP, LH>();
     // one slot past the last box's first for each of its chunks (its list may end inside a chunk)
-    const int64_t slots = mx_first_slot(Ls.n_m2l, Ls.n_m2l_targets, mx_chunk<CAP, LH>());
-    const int64_t want = (slots + NW - 1) / NW;
+    const int64_t slots = mx_first_slot(Ls.n_m2l, Ls.n_m2l_targets, S), len = (LH ? 4 : 2) * nh(p);
+    const int64_t span = (st.n_branches + S - 1) / S;
+    const int64_t room = std::max<int64_t>(MX_PART_BYTES / (int64_t)(len * sizeof(double)), 2 * span);
+    const int64_t pass = slots <= room ? slots : room - span, held = std::min(slots, room);
+    C.m2l_part.resize((size_t)(held * len));
+    const int64_t want = (held + NW - 1) / NW;
     const unsigned grid = (unsigned)std::max<int64_t>(1, std::min<int64_t>(want, (int64_t)std::max(per_cu, 1) * C.n_cu));
     // The counter is one address for all 8 XCDs and takes an increment about every 14 ns. Up to cap 12 a slot is less work
     // than that over 2048-3072 wavefronts (4M Plummer sphere, order 8: 18.3 ms with one increment per slot, 9.0 ms with
     // several), so a wavefront takes two to sixteen at a time, a sixth of its share; above, a slot is ten times as long
     // (1M ring, order cap 20: 20.3 ms with one, 21.8 ms with several). With a wavefront for every slot there is no counter
     // (grab 0): a small launch otherwise spends a third of its time on it.
-    const int64_t waves = (int64_t)grid * NW, share = slots / waves;
-    const int grab = slots <= waves ? 0 : CAP <= 12 && share >= 4 ? (int)std::max<int64_t>(2, std::min<int64_t>(16, share / 6)) : 1;
-    C.m2l_part.resize((size_t)slots * ((LH ? 4 : 2) * nh(p)));
-    kfn<<<grid, 64 * NW, sh, C.stream>>>(Ls.m2l_targets.data(), Ls.m2l_offsets.data(), Ls.m2l_s.data(), tt_dst.branches.data(),
-                                         st.branches.data(), st.expansions.data(), tt_dst.expansions.data(), C.m2l_part.data(),
-                                         (int)Ls.n_m2l_targets, slots, grab, p, pe, E, perm, Ls.m2l_order.data(), flags,
-                                         Ls.track_box_ok ? const_cast<int32_t*>(Ls.m2l_box_ok.data()) : nullptr, tb);
-    LAUNCH_CHECK();
-    k_m2l_mx_sum<CAP, LH><<<(unsigned)Ls.n_m2l_targets, 256, 0, C.stream>>>(Ls.m2l_targets.data(), Ls.m2l_offsets.data(),
-                                                                          tt_dst.expansions.data(), C.m2l_part.data(), p, pe);
-    LAUNCH_CHECK();
+    const int64_t waves = (int64_t)grid * NW, share = held / waves;
+    const int grab = held <= waves ? 0 : CAP <= 12 && share >= 4 ? (int)std::max<int64_t>(2, std::min<int64_t>(16, share / 6)) : 1;
+    for (int64_t w0 = 0; w0 < slots; w0 += pass) {
+        const int64_t w1 = std::min(slots, w0 + pass);
+        kfn<<<grid, 64 * NW, sh, C.stream>>>(Ls.m2l_targets.data(), Ls.m2l_offsets.data(), Ls.m2l_s.data(), tt_dst.branches.data(),
+                                             st.branches.data(), st.expansions.data(), tt_dst.expansions.data(), C.m2l_part.data(),
+                                             (int)Ls.n_m2l_targets, (int)w0, (int)w1, (int)std::min(slots, w1 + span), grab, p, pe,
+                                             E, perm, Ls.m2l_order.data(), flags,
+                                             Ls.track_box_ok ? const_cast<int32_t*>(Ls.m2l_box_ok.data()) : nullptr, tb);
+        LAUNCH_CHECK();
+        k_m2l_mx_sum<CAP, LH><<<(unsigned)Ls.n_m2l_targets, 256, 0, C.stream>>>(
+            Ls.m2l_targets.data(), Ls.m2l_offsets.data(), tt_dst.expansions.data(), C.m2l_part.data(), (int)w0, (int)w1, p, pe, flags);
+        LAUNCH_CHECK();
+    }
 }
 
 
