@@ -234,6 +234,8 @@ __host__ __device__ inline int data_per_body(int kernel) {
 // rows after [x, y, z, radius] kept with every sorted body: strengths (and panel vertices)
 inline int strength_dims(int kernel) { return kernel == FMMHIP_POINT_SOURCE ? 1 : data_per_body(kernel) - 4; }
 inline bool valid_kernel(int kernel) { return kernel >= FMMHIP_POINT_SOURCE && kernel <= FMMHIP_PANEL_SOURCE_DIPOLE_QUAD; }
+// doubles of a panel's nearfield record (PanelStage, panels.hpp): an odd number
+__host__ __device__ constexpr int panel_record_doubles(int vertices) { return (15 + 5 * vertices) | 1; }
 // has_vector_potential (test/vortex.jl:145-147): Lamb-Helmholtz chi expansions
 inline bool has_vector_potential(int kernel) {
     return kernel == FMMHIP_POINT_VORTEX || kernel == FMMHIP_VORTEX_GAUSSIAN || kernel == FMMHIP_POINT_SOURCE_VORTEX;
@@ -281,6 +283,10 @@ size_t direct_scratch_bytes();
 // expansions.hip
 void ensure_tables(Context& C, int p);
 void free_tables(Tables* t);
+// matrix-core M2L (m2l_mx_gpu.hpp): list entries per chunk at an order (an order cap's orders have one), and the bytes
+// that the partial expansions of a launch take at most
+constexpr int m2l_chunk(int p, bool lh) { return (p <= 12 ? 1 : 2) * (lh ? 8 : 16); }
+static constexpr int64_t M2L_PART_BYTES = (int64_t)2 << 30;
 // sbr: the source tree's branches with one system's leaf ranges (several systems in one tree), or null
 void run_p2m(Context& C, int kernel, Tree& st, int p, const Branch* sbr = nullptr);
 void run_m2m(Context& C, Tree& st, int p, bool LH);

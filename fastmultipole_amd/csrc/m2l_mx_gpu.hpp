@@ -124,19 +124,14 @@ static size_t mx_lds_bytes(int nw) {
 // `part` and k_m2l_mx_sum adds them in chunk order. S depends on the cap alone, never on the size of the problem, so a
 // box's sum is the same to the last bit whatever is evaluated beside it. S is a few batches: a chunk's partial
 // expansion (7.4 KB at cap 20) is written and read once per S interactions, 0.3 ms of the 1M ring's 30 ms.
-template <int CAP, bool LH>
-constexpr int mx_chunk() {
-    return (CAP <= 12 ? 1 : 2) * (LH ? 8 : 16);
-}
 __host__ __device__ inline int64_t mx_first_slot(int64_t l0, int64_t box, int S) { return l0 / S + box; }
 
-// Bytes of partial expansions at most. The slots of larger launches are taken in passes: the pass from w0 to w1 takes
-// every chunk of the boxes whose first slot lies in it, up to `span` slots past w1 (a list holds a source branch once, so
-// its chunks are no more than n_branches / S), and k_m2l_mx_sum adds them before the next pass. A box is summed whole in
-// one pass, so its sum does not depend on where the passes end. One pass for 4M bodies at order 8 (1.1 GB) or the 1M ring
-// at order 20 (1.0 GB); without a bound 2.5M uniform vortices at order 20 (37M interactions) took 20.7 GiB, and 428 ms
-// against 430 ms in ten passes.
-static constexpr int64_t MX_PART_BYTES = (int64_t)2 << 30;
+// The partial expansions take M2L_PART_BYTES at most. The slots of larger launches are taken in passes: the pass from w0 to
+// w1 takes every chunk of the boxes whose first slot lies in it, up to `span` slots past w1 (a list holds a source branch
+// once, so its chunks are no more than n_branches / S), and k_m2l_mx_sum adds them before the next pass. A box is summed
+// whole in one pass, so its sum does not depend on where the passes end. One pass for 4M bodies at order 8 (1.1 GB) or
+// the 1M ring at order 20 (1.0 GB); without a bound 2.5M uniform vortices at order 20 (37M interactions) took 20.7 GiB,
+// and 428 ms against 430 ms in ten passes.
 
 // the box whose slots hold slot w: the last one whose first slot is not above w (64 candidates per step)
 __device__ inline int mx_box_of(const int64_t* __restrict__ m2l_offsets, int n_boxes, int64_t w, int S, int lane) {
@@ -214,7 +209,7 @@ __global__ __launch_bounds__(64 * NW, CAP <= 12 ? 2 : 1) void k_m2l_mx(const int
     const int64_t HE4 = 4 * (int64_t)nh(PE);
     const int lane = lane_id();
     int pmax = 0, okf = 1;
-    constexpr int S = mx_chunk<CAP, LH>();
+    constexpr int S = m2l_chunk(CAP, LH);
     int slot = -1, left = 0, box = 0;
     int64_t lb = 0, le = 0;
     for (;;) {
@@ -290,7 +285,7 @@ __global__ __launch_bounds__(256) void k_m2l_mx_sum(const int32_t* __restrict__ 
                                                     const int64_t* __restrict__ m2l_offsets, double* __restrict__ tex,
                                                     const double* __restrict__ part, int w0, int w1, int P, int PE,
                                                     int32_t* __restrict__ flags) {
-    constexpr int S = mx_chunk<CAP, LH>(), NC = LH ? 4 : 2;
+    constexpr int S = m2l_chunk(CAP, LH), NC = LH ? 4 : 2;
     const int box = blockIdx.x;
     if (box == 0 && threadIdx.x == 0) flags[2] = 0;
     const int64_t l0 = m2l_offsets[box], l1 = m2l_offsets[box + 1], first = mx_first_slot(l0, box, S);
@@ -315,11 +310,11 @@ static void launch_m2l_mx(Context& C, int p, int pe, const Lists& Ls, const Tree
     int per_cu = 0;
     HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(kfn), 64 * NW, sh));
     if (!C.n_cu) HIP_CHECK(hipDeviceGetAttribute(&C.n_cu, hipDeviceAttributeMultiprocessorCount, C.device));
-    constexpr int S = mx_chunk<CAP, LH>();
+    constexpr int S = m2l_chunk(CAP, LH);
     // one slot past the last box's first for each of its chunks (its list may end inside a chunk)
     const int64_t slots = mx_first_slot(Ls.n_m2l, Ls.n_m2l_targets, S), len = (LH ? 4 : 2) * nh(p);
     const int64_t span = (st.n_branches + S - 1) / S;
-    const int64_t room = std::max<int64_t>(MX_PART_BYTES / (int64_t)(len * sizeof(double)), 2 * span);
+    const int64_t room = std::max<int64_t>(M2L_PART_BYTES / (int64_t)(len * sizeof(double)), 2 * span);
     const int64_t pass = slots <= room ? slots : room - span, held = std::min(slots, room);
     C.m2l_part.resize((size_t)(held * len));
     const int64_t want = (held + NW - 1) / NW;

@@ -33,6 +33,8 @@ template <int NV> struct PanelStage {
     // an odd number of doubles: lanes on consecutive panels of a tile read different LDS banks
     double pad[(14 + 5 * NV) % 2 == 0 ? 1 : 2];
 };
+static_assert(sizeof(PanelStage<3>) == 8 * panel_record_doubles(3) && sizeof(PanelStage<4>) == 8 * panel_record_doubles(4),
+              "the request server's estimate counts these records");
 
 // panel j of the sorted arrays (rows after radius: NSTR strengths, v1, v2, ...) into a stage
 template <int NV, int NSTR = 1>

@@ -53,7 +53,8 @@ struct Job {
 };
 
 // HBM estimate of one request (bytes): body arrays and outputs, two trees with
-// their expansions, lists, and for a solve the influence blocks
+// their expansions, lists, the M2L's partial expansions (none at the fixed orders of the lane
+// kernel), panel records, and for a solve the influence blocks
 double footprint_bytes(const fmmhip_request& r) {
     const double n = (double)std::max<int64_t>(1, r.n);
     const int p = std::max(1, r.options.expansion_order);
@@ -63,7 +64,14 @@ double footprint_bytes(const fmmhip_request& r) {
     double b = n * 8.0 * (fmmhip::data_per_body(r.kernel) + 3 + 13 + 16 + 24);
     b += 2.0 * branches * (sizeof(fmmhip::Branch) + 32.0 * H);
     b += branches * 400.0 * 16.0;
-    b += branches * 6.0 * 32.0 * H;   // partial expansions of the M2L's list chunks
+    if (r.options.error_kind != FMMHIP_ERR_NONE || p > 4) {
+        // about 150 interactions per box (measured: 135 of uniform sources at acceptance 0.4), a slot more than its full
+        // chunks for each box, up to the workspace's bound; the buffer's slack of an eighth
+        const bool lh = fmmhip::has_vector_potential(r.kernel);
+        const double slots = branches * (150.0 / fmmhip::m2l_chunk(p, lh) + 1.0);
+        b += 1.125 * std::min(slots * (lh ? 32.0 : 16.0) * H, (double)fmmhip::M2L_PART_BYTES);
+    }
+    if (fmmhip::is_panel(r.kernel)) b += 1.125 * n * 8.0 * fmmhip::panel_record_doubles(fmmhip::panel_vertices(r.kernel));
     if (r.kind == FMMHIP_REQUEST_SOLVE) b += n * leaf * 8.0 * 30.0 + n * 8.0 * 40.0;
     return b;
 }

@@ -6,6 +6,8 @@ deterministic: integer atomics only); FastGaussSeidel solves within 1e-10 relati
 solve with the same sweep count (a sweep level adds right-hand-side updates with floating-point
 atomics, whose order varies run to run). The single calls are themselves pinned against the
 oracle by the parity and FastGaussSeidel tests."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -129,6 +131,41 @@ def test_server_budget_serialises_requests():
     spans.sort()
     for (s0, e0), (s1, _) in zip(spans, spans[1:]):
         assert s1 >= e0, spans     # no overlap: each starts after the previous ended
+
+
+def _free_bytes():
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert _lib.load().hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0   # the runtime the library is linked to
+    return free.value
+
+
+def test_admission_estimate_counts_the_m2l_workspace_and_the_panel_records(monkeypatch):
+    """The estimate's share of the M2L's partial expansions is at least what they take: the difference of two orders' estimates,
+    the lower without such a workspace, less the difference of their two trees' expansions. A panel request's is
+    its rows and records above a point request's."""
+    print("[gpu] server admission estimate", flush=True)
+    n, leaf, mac = 400000, 20, 0.5
+    rows = W.uniform_vortices(n, seed=31)
+    with F.Server(n_slots=1) as server:
+        def estimate(kernel, r, **kw):
+            return server.wait(server.submit_fmm(_Rows(kernel, r), multipole_acceptance=mac, **kw))[2]["footprint_bytes"]
+        fp = {p: estimate(_lib.POINT_VORTEX, rows, leaf_size=leaf, expansion_order=p) for p in (4, 12)}
+        panels, _ = W.sphere_panels(20, quads=True)
+        points = estimate(_lib.POINT_SOURCE, W.uniform_sources(len(panels), seed=32), leaf_size=30)
+        fp_panels = estimate(_lib.PANEL_SOURCE_QUAD, panels, leaf_size=30)
+    ev = F.Evaluation()
+    ev.set_systems(_lib.POINT_VORTEX, None, rows)
+    for engine in ("wave", "mx"):   # the same handle: all other buffers have their size after the first
+        monkeypatch.setenv("FMMHIP_M2L_KERNEL", engine)
+        before = _free_bytes()
+        ev.fmm(F.make_options(expansion_order=12, leaf_size_source=leaf, multipole_acceptance=mac))
+        workspace = before - _free_bytes()
+    ev.close()
+    coefficients = lambda p: (p + 1) * (p + 2) // 2
+    branches = 2.3 * n / leaf + 64
+    assert workspace > 1e9
+    assert fp[12] - fp[4] - 2 * branches * 32 * (coefficients(12) - coefficients(4)) >= workspace
+    assert fp_panels - points >= len(panels) * 8 * ((17 - 5) + 35)
 
 
 def test_server_rejects_bad_requests():
