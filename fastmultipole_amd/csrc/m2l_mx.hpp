@@ -46,8 +46,8 @@
 // bits and an order decision sitting on the tolerance can flip.
 //
 // The engine is written against a backend B (per-lane value types, cross-lane moves, the MFMA) so the
-// same source runs on the GPU (backend in expansions.hip) and lane by lane on the CPU (the emulation
-// used by the tests). It is plain C++ apart from the backend.
+// same source runs on the GPU (backend in m2l_mx_gpu.hpp) and lane by lane on the CPU (the emulation
+// used by the tests), with the same tables and scratch in the same order. It is plain C++ apart from the backend.
 #pragma once
 #include <cstdint>
 #include <type_traits>
@@ -70,10 +70,10 @@ template <int n>
 struct LO {   // LOFF(n) as a constant (register arrays need compile-time indices)
     static constexpr int v = LOFF(n);
 };
-constexpr int AST(int n) { return (n + 2) & ~1; }            // row length of the dense pi/2 table of degree n
+constexpr int AST(int n) { return (n + 2) & ~1; }            // row length of degree n in the dense pi/2 tables (host_dense_A)
 constexpr int ABASE(int n) { return (n * (n + 1) * (2 * n + 1)) / 6 + ((n + 1) / 2) * ((n + 1) / 2); }
-constexpr int ALEN(int cap) { return ABASE(cap + 1); }
-// zero-padded pi/2 table: degree n as (KE + KO)^2 blocks of 4x4 at PBASE(n), rows and columns by parity (E groups, then O)
+// zero-padded pi/2 table: degree n as (KE + KO)^2 blocks of 4x4 at PBASE(n), rows and columns by parity (E groups, then O).
+// Rows and columns past the degree are zero in every product, so no row of a rotation needs a mask.
 constexpr int PBASE(int n) { return n <= 0 ? 0 : PBASE(n - 1) + 16 * (KE(n - 1) + KO(n - 1)) * (KE(n - 1) + KO(n - 1)); }
 constexpr int PLEN(int cap) { return PBASE(cap + 1); }
 constexpr int imin(int a, int b) { return a < b ? a : b; }
@@ -87,40 +87,17 @@ MX_FN void sfor(F&& f) {
     }
 }
 
-// d += A B on four blocks of 4x4x4: lane l supplies A(l % 4, l / 16) (the same in every block), B(l / 16, l % 16) and
-// holds D(l / 16, l % 16). A backend without the instruction takes the first four rows of the 16x16x4 product.
-template <class B, class = void>
-struct Prod {
-    MX_FN static void add(const typename B::V& a, const typename B::V& b, typename B::V& d) {
-        typename B::V4 t = B::zero4();
-        B::set4(t, 0, d);
-        B::mfma(a, b, t);
-        d = B::get4(t, 0);
-    }
-};
-template <class B>
-struct Prod<B, std::void_t<decltype(&B::mfma4)>> {
-    MX_FN static void add(const typename B::V& a, const typename B::V& b, typename B::V& d) { d = B::mfma4(a, b, d); }
-};
-
-// A backend with `padded` holds the pi/2 tables in the zero-padded form. Rows and columns past the degree are then zero in
-// every product, so no row of a rotation needs a mask; in the dense form such entries belong to other rows.
-template <class B, class = void>
-struct Padded : std::false_type {};
-template <class B>
-struct Padded<B, std::void_t<typename B::padded>> : std::true_type {};
-
 // Shared tables (LDS on the GPU), for degrees 0..CAP; per (n, m) tables are indexed mnh(n - 1) + m.
 struct Tabs {
-    const double* A;     // dense pi/2 tables: degree n at ABASE(n), row-major, rows of AST(n); or the padded form (PBASE)
-    const double* zin;   // zeta input scale (multipole rotation)
-    const double* zoh;   // half the zeta output scale
-    const double* ein;   // eta input scale (local rotation)
-    const double* eoh;   // half the eta output scale
-    const double* Mt;    // multipole power normalisation
-    const double* Lt;    // local power normalisation
-    const double* tf;    // per degree n: 1/(n-1)!, (n+1)!
-    const double* i0;    // per degree n: 1 / Mt(n, 0), 1 / Lt(n, 0)
+    double* A;     // zero-padded pi/2 tables
+    double* zin;   // zeta input scale (multipole rotation)
+    double* zoh;   // half the zeta output scale
+    double* ein;   // eta input scale (local rotation)
+    double* eoh;   // half the eta output scale
+    double* Mt;    // multipole power normalisation
+    double* Lt;    // local power normalisation
+    double* tf;    // per degree n: 1/(n-1)!, (n+1)!
+    double* i0;    // per degree n: 1 / Mt(n, 0), 1 / Lt(n, 0)
 };
 
 // per-wavefront scratch
@@ -130,6 +107,37 @@ struct Wave {
     double* acc;   // mnh(CAP) x NC: the target box's local expansion, summed over the wave's interactions
     double* F;     // BP x (2 CAP + 1): z-translation factors j! / t^(j+1) of each slot
 };
+
+// Where they lie: the tables, then each wavefront's scratch. Rows past a degree are read unmasked (they are multiplied by
+// zero): past a degree's row of an (n, m) table into the next degree or the next table, past a slot's phases into the
+// next slot's, and past the last slot's eim into cs, past its cs into F. Every double so read is written before.
+template <int CAP>
+constexpr int shared_doubles() {
+    return PLEN(CAP) + 6 * mnh(CAP) + 4 * (CAP + 1);
+}
+template <int CAP>
+MX_FN Tabs tabs(double* lds) {
+    constexpr int H = mnh(CAP);
+    double* t = lds + PLEN(CAP);
+    return {lds, t, t + H, t + 2 * H, t + 3 * H, t + 4 * H, t + 5 * H, t + 6 * H, t + 6 * H + 2 * (CAP + 1)};
+}
+template <int CAP, bool LH>
+constexpr int wave_doubles() {
+    return (LH ? 4 : 2) * mnh(CAP) + 4 * (LH ? 8 : 16) * (CAP + 1) + (LH ? 8 : 16) * (2 * CAP + 1);
+}
+template <int CAP, bool LH>
+MX_FN Wave wave(double* w) {
+    constexpr int A = (LH ? 4 : 2) * mnh(CAP), E = 2 * (LH ? 8 : 16) * (CAP + 1);
+    return {w + A, w + A + E, w, w + A + 2 * E};
+}
+// entry t of degree n's blocks in the padded table, from the dense tables
+template <class D>
+MX_FN double padded(const D* Ad, int n, int t) {
+    const int ke = KE(n), nb = ke + KO(n);
+    const int rq = t / (16 * nb), kq = (t >> 4) % nb, i = (t >> 2) & 3, q = t & 3;
+    const int row = (rq < ke ? 8 * rq : 8 * (rq - ke) + 1) + 2 * i, col = (kq < ke ? 8 * kq : 8 * (kq - ke) + 1) + 2 * q;
+    return row <= n && col <= n ? Ad[ABASE(n) + row * AST(n) + col] : 0.0;
+}
 
 // BP consecutive entries b0 .. b0 + nb - 1 of the target box's part of the M2L list, taken in the
 // order perm gives (list indices; null: list order)
@@ -150,8 +158,8 @@ struct Box {
     int BE;         // the order settles at the passing degree (1) or one below (0)
 };
 
-// EK: 0 fixed orders only, 1 error-controlled only, -1 either (Box::kind says which)
-template <class B, int CAP, bool LH, int EK = -1>
+// ERR: error-controlled orders (Box::kind 1 to 3), else the fixed order P (kind 0)
+template <class B, int CAP, bool LH, bool ERR>
 struct Engine {
     using V = typename B::V;
     using I = typename B::I;
@@ -160,7 +168,6 @@ struct Engine {
     static constexpr int NP = LH ? 2 : 1;    // potentials
     static constexpr int NC = 2 * NP;        // real components per coefficient
     static constexpr int BP = 16 / NP;
-    static constexpr bool PAD = Padded<B>::value;
     static constexpr int NL = NLREG(CAP);    // registers of the local expansion, per real or imaginary part
     static constexpr int NS = CAP + 1;   // slot-table entries
     static constexpr int NF = 2 * CAP + 1;   // translation factors per slot
@@ -264,43 +271,36 @@ struct Engine {
         B::wsync();
     }
 
-    // One rotation of degree n (compile-time) of the coefficient vector u (input scale applied, row 0 halved, rows
-    // m > n zero): out as in the header, without the factor 4 w (in the slot tables) and with rows m > n zero. sigma = +1
-    // multipole (zeta), -1 local (eta). In the dense form the A operands are read unmasked: entries outside the degree's
-    // table multiply zero rows of u (first products) or rows of R that are set to zero (second products), or land in
-    // output rows m > n, which are discarded. In the padded form these rows may hold any finite value.
+    // One rotation of degree n (compile-time) of the coefficient vector u (input scale applied, row 0 halved): out as in
+    // the header, without the factor 4 w (in the slot tables). sigma = +1 multipole (zeta), -1 local (eta). Rows m > n of u
+    // may hold any finite value (the padded table's columns are zero there); rows m > n of the result are zero.
     template <int n>
     MX_FN static void rotate(const Tabs& T, const Wave& W, const double* gout, double sigma, I c, I q, I s,
                              const V (&uEr)[imax(KE(n), 1)], const V (&uEi)[imax(KE(n), 1)], const V (&uOr)[imax(KO(n), 1)],
                              const V (&uOi)[imax(KO(n), 1)], V (&oEr)[imax(KE(n), 1)], V (&oEi)[imax(KE(n), 1)],
                              V (&oOr)[imax(KO(n), 1)], V (&oOi)[imax(KO(n), 1)]) {
-        constexpr int ke = KE(n), ko = KO(n), st = AST(n), ab = ABASE(n);
+        constexpr int ke = KE(n), ko = KO(n);
         const I q2 = q * 2, i2 = (c & 3) * 2;
-        const I lo = i2 * st + q2;
         // A block of rows 8 r + pr + 2 (lane % 4) and columns 8 k + pk + 2 (lane / 16)
         auto blk = [&](auto R, auto PR, auto KK, auto PK) {
-            constexpr int r0 = 8 * decltype(R)::value + decltype(PR)::value, k0 = 8 * decltype(KK)::value + decltype(PK)::value;
-            if constexpr (PAD) {
-                constexpr int rq = decltype(R)::value + (decltype(PR)::value ? ke : 0);
-                constexpr int kq = decltype(KK)::value + (decltype(PK)::value ? ke : 0);
-                return B::lds(T.A, i2 * 2 + q + (PBASE(n) + (rq * (ke + ko) + kq) * 16));
-            } else if constexpr (ab + (r0 + 6) * st + k0 + 6 < ALEN(CAP)) return B::lds(T.A, lo + (ab + r0 * st + k0));
-            else return B::lds(T.A, B::mini(i2 + r0, n) * st + B::mini(q2 + k0, n) + ab);
+            constexpr int rq = decltype(R)::value + (decltype(PR)::value ? ke : 0);
+            constexpr int kq = decltype(KK)::value + (decltype(PK)::value ? ke : 0);
+            return B::lds(T.A, i2 * 2 + q + (PBASE(n) + (rq * (ke + ko) + kq) * 16));
         };
         using C0 = std::integral_constant<int, 0>;
         using C1 = std::integral_constant<int, 1>;
         const I sb = s * (NS * 2);
-        auto okrow = [&](auto par, auto RI) { return q2 + (8 * decltype(RI)::value + decltype(par)::value) <= n; };
         sfor<0, ke>([&](auto AA) { oEr[decltype(AA)::value] = V(0.0); oEi[decltype(AA)::value] = V(0.0); });
         sfor<0, imax(ko, 1)>([&](auto AA) { oOr[decltype(AA)::value] = V(0.0); oOi[decltype(AA)::value] = V(0.0); });
+        auto add = [](const V& a, const V& b, V& d) { d = B::mfma4(a, b, d); };
         // the v of one register (parity par): first products, combination, second products
         auto half = [&](auto par, auto VI) {
             constexpr int pv = decltype(par)::value, vi = decltype(VI)::value, v0 = 8 * vi + pv;
             constexpr bool even = ((n + pv) & 1) == 0;   // n + v even
             V se = V(0.0), so = V(0.0);   // the needed parts of S_E and S_O
-            sfor<0, ke>([&](auto EE) { Prod<B>::add(blk(VI, par, EE, C0()), even ? uEr[decltype(EE)::value] : uEi[decltype(EE)::value], se); });
-            sfor<0, ko>([&](auto OO) { Prod<B>::add(blk(VI, par, OO, C1()), even ? uOi[decltype(OO)::value] : uOr[decltype(OO)::value], so); });
-            const I vr = (PAD || v0 + 6 <= n) ? q2 + v0 : B::mini(q2 + v0, n);
+            sfor<0, ke>([&](auto EE) { add(blk(VI, par, EE, C0()), even ? uEr[decltype(EE)::value] : uEi[decltype(EE)::value], se); });
+            sfor<0, ko>([&](auto OO) { add(blk(VI, par, OO, C1()), even ? uOi[decltype(OO)::value] : uOr[decltype(OO)::value], so); });
+            const I vr = q2 + v0;
             const I ci = sb + vr * 2;
             const V cv = B::lds(W.cs, ci), sv = B::lds(W.cs, ci + 1) * sigma;
             V re, ro;
@@ -311,58 +311,41 @@ struct Engine {
                 re = B::fma(-sv, so, cv * se);
                 ro = -B::fma(cv, so, sv * se);
             }
-            if constexpr (!PAD && v0 + 6 > n) {
-                const M ok = okrow(par, VI);
-                re = B::sel(ok, re, V(0.0));
-                ro = B::sel(ok, ro, V(0.0));
-            }
             sfor<0, ke>([&](auto AA) {
                 constexpr int a = decltype(AA)::value;
-                Prod<B>::add(blk(AA, C0(), VI, par), re, even ? oEr[a] : oEi[a]);
+                add(blk(AA, C0(), VI, par), re, even ? oEr[a] : oEi[a]);
             });
             sfor<0, ko>([&](auto AA) {
                 constexpr int a = decltype(AA)::value;
-                Prod<B>::add(blk(AA, C1(), VI, par), ro, even ? oOi[a] : oOr[a]);
+                add(blk(AA, C1(), VI, par), ro, even ? oOi[a] : oOr[a]);
             });
         };
         sfor<0, ke>([&](auto VI) { half(C0(), VI); });
         sfor<0, ko>([&](auto VI) { half(C1(), VI); });
         auto out = [&](auto par, auto RI, V& xr, V& xi) {
             constexpr int m0 = 8 * decltype(RI)::value + decltype(par)::value;
-            if constexpr (PAD || m0 + 6 <= n) {
-                const V g = B::lds(gout, q2 + (m0 + mnh(n - 1)));
-                xr = g * xr;
-                xi = g * xi;
-            } else {
-                const M ok = q2 + m0 <= n;
-                const V g = B::lds(gout, B::mini(q2 + m0, n) + mnh(n - 1));
-                xr = B::sel(ok, g * xr, V(0.0));
-                xi = B::sel(ok, g * xi, V(0.0));
-            }
+            const V g = B::lds(gout, q2 + (m0 + mnh(n - 1)));
+            xr = g * xr;
+            xi = g * xi;
         };
         sfor<0, ke>([&](auto EE) { out(C0(), EE, oEr[decltype(EE)::value], oEi[decltype(EE)::value]); });
         sfor<0, ko>([&](auto OO) { out(C1(), OO, oOr[decltype(OO)::value], oOi[decltype(OO)::value]); });
     }
 
-    // the source coefficients of degree n for this lane's rows (E registers, then O); rows m > n are zero, or row n's in
-    // the padded form
+    // the source coefficients of degree n for this lane's rows (E registers, then O); rows m > n are row n's
     template <int n>
     MX_FN static void fetch(const PV& src, I q, I pot, V (&xr)[NX], V (&xi)[NX]) {
         auto one = [&](auto par, auto RI, V& r, V& i) {
             constexpr int m0 = 8 * decltype(RI)::value + decltype(par)::value;
             const I at = (q * 2) * 4 + pot * 2;
             constexpr int k0 = (m0 + mnh(n - 1)) * 4;
-            if constexpr (PAD && m0 + 6 > n) {
+            if constexpr (m0 + 6 > n) {
                 const I last = B::mini(q * 2 + m0, n) * 4 + pot * 2;
-                r = B::gldp(src, last + mnh(n - 1) * 4, M(true));
-                i = B::gldp(src, last + (mnh(n - 1) * 4 + 1), M(true));
-            } else if constexpr (m0 + 6 <= n) {
-                r = B::gldp(src, at + k0, M(true));
-                i = B::gldp(src, at + (k0 + 1), M(true));
+                r = B::gldp(src, last + mnh(n - 1) * 4);
+                i = B::gldp(src, last + (mnh(n - 1) * 4 + 1));
             } else {
-                const M ok = q * 2 + m0 <= n;
-                r = B::gldp(src, at + k0, ok);
-                i = B::gldp(src, at + (k0 + 1), ok);
+                r = B::gldp(src, at + k0);
+                i = B::gldp(src, at + (k0 + 1));
             }
         };
         sfor<0, KE(n)>([&](auto EE) { one(std::integral_constant<int, 0>(), EE, xr[decltype(EE)::value], xi[decltype(EE)::value]); });
@@ -388,7 +371,7 @@ struct Engine {
         const I s0 = LH ? (c0 >> 1) & 7 : c0, pot0 = LH ? c0 & 1 : I(0);
         const M valid = s0 < Bt.nb;
         const int P = X.P;
-        const bool err = EK < 0 ? X.kind != 0 : EK != 0;
+        constexpr bool err = ERR;
 
         // an empty slot reads the batch's first interaction; its phases are zero (slot_tables)
         const I li = entry(Bt, s0, valid);
@@ -444,11 +427,11 @@ struct Engine {
             const bool power = err && X.kind >= 2;
             auto load = [&](auto par, auto RI, V& ur, V& ui) {
                 constexpr int pr = decltype(par)::value, ri = decltype(RI)::value, m0 = 8 * ri + pr;
-                const I mi = (PAD || m0 + 6 <= k) ? q2 + m0 : B::mini(q2 + m0, k);
+                const I mi = q2 + m0;
                 const V xr = xcr[(pr ? ke : 0) + ri], xi = xci[(pr ? ke : 0) + ri];
                 if (power) {
                     V nt = B::lds(T.Mt, mi + mnh(k - 1));
-                    if constexpr (PAD && m0 + 6 > k) nt = B::sel(q2 + m0 <= k, nt, V(0.0));
+                    if constexpr (m0 + 6 > k) nt = B::sel(q2 + m0 <= k, nt, V(0.0));
                     pw_t = B::fma(B::fma(xr, xr, xi * xi) * nt, nt, pw_t);
                 }
                 const I ei = sb2 + mi * 2;
@@ -676,9 +659,7 @@ struct Engine {
             auto scale = [&](auto par, auto RI, V& ur, V& ui) {
                 constexpr int pr = decltype(par)::value, ri = decltype(RI)::value, m0 = 8 * ri + pr;
                 constexpr int at = LO<n>::v + (pr ? ke : 0) + ri;
-                const I mi = (PAD || m0 + 6 <= n) ? q2 + m0 : B::mini(q2 + m0, n);
-                V g = B::lds(T.ein, mi + mnh(n - 1));
-                if (!PAD && m0 + 6 > n) g = B::sel(q2 + m0 <= n, g, V(0.0));
+                V g = B::lds(T.ein, q2 + (m0 + mnh(n - 1)));
                 if (err) g = B::sel(on, g, V(0.0));
                 ur = g * Lr[at];
                 ui = g * Li[at];
@@ -691,7 +672,7 @@ struct Engine {
             auto store = [&](auto par, auto RI, const V& xr, const V& xi) {
                 constexpr int m0 = 8 * decltype(RI)::value + decltype(par)::value;
                 const I m = q2 + m0;
-                const I ei = sb2 + ((PAD || m0 + 6 <= n) ? m : B::mini(m, n)) * 2;
+                const I ei = sb2 + m * 2;
                 const V er = B::lds(W.eim, ei), eimg = B::lds(W.eim, ei + 1);
                 // back_rotate_z! (src/rotate.jl:584-616)
                 const V zr = B::template slotsum<NP>(B::fma(xr, er, xi * eimg));

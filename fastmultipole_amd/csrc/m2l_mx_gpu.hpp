@@ -31,7 +31,6 @@ struct MxGpu {
     using I = int;
     using M = bool;
     using PV = const double*;
-    struct padded;   // the pi/2 tables are held in the zero-padded form
     static __device__ __forceinline__ I lane() { return (int)(threadIdx.x & 63); }
     static __device__ __forceinline__ V sel(M m, V a, V b) { return m ? a : b; }
     static __device__ __forceinline__ I seli(M m, I a, I b) { return m ? a : b; }
@@ -84,11 +83,7 @@ struct MxGpu {
         return r;
     }
     static __device__ __forceinline__ PV ptr(const double* base, I js, int64_t stride) { return base + (int64_t)js * stride; }
-    static __device__ __forceinline__ V gldp(PV p, I i, M ok) {
-        V r = 0.0;
-        if (ok) r = p[i];
-        return r;
-    }
+    static __device__ __forceinline__ V gldp(PV p, I i) { return p[i]; }
     static __device__ __forceinline__ V lds(const double* p, I i) { return p[i]; }
     static __device__ __forceinline__ void lds_st(double* p, I i, V x, M ok) {
         if (ok) p[i] = x;
@@ -103,16 +98,8 @@ struct MxGpu {
 };
 
 template <int CAP, bool LH>
-__host__ __device__ constexpr int mx_wave_doubles() {
-    return (LH ? 4 : 2) * nh(CAP) + 4 * (LH ? 8 : 16) * (CAP + 1) + (LH ? 8 : 16) * (2 * CAP + 1);
-}
-template <int CAP>
-__host__ __device__ constexpr int mx_shared_doubles() {
-    return mx::PLEN(CAP) + 6 * nh(CAP) + 4 * (CAP + 1);
-}
-template <int CAP, bool LH>
 static size_t mx_lds_bytes(int nw) {
-    return sizeof(double) * (size_t)(mx_shared_doubles<CAP>() + nw * mx_wave_doubles<CAP, LH>());
+    return sizeof(double) * (size_t)(mx::shared_doubles<CAP>() + nw * mx::wave_doubles<CAP, LH>());
 }
 
 // Work items. A target box's list entries are cut into chunks of S (the last one shorter), and a wavefront takes one
@@ -165,47 +152,34 @@ __global__ __launch_bounds__(64 * NW, CAP <= 12 ? 2 : 1) void k_m2l_mx(const int
                                                     const int32_t* __restrict__ perm, int32_t* __restrict__ orders,
                                                     int32_t* __restrict__ flags, int32_t* __restrict__ box_ok,
                                                     TablePtrs tb) {
-    using Eng = mx::Engine<MxGpu, CAP, LH, ERR ? 1 : 0>;
+    using Eng = mx::Engine<MxGpu, CAP, LH, ERR>;
     constexpr int H = nh(CAP), NC = Eng::NC, BP = Eng::BP, NS = CAP + 1;
     extern __shared__ double lds[];
-    double* A = lds;
-    double* zin = A + mx::PLEN(CAP);
-    double* zoh = zin + H;
-    double* ein = zoh + H;
-    double* eoh = ein + H;
-    double* Mt = eoh + H;
-    double* Lt = Mt + H;
-    double* tf = Lt + H;
+    const mx::Tabs T = mx::tabs<CAP>(lds);
+#pragma unroll CAP <= 12 ? CAP + 1 : 1
     for (int n = 0, at = 0; n <= CAP; ++n) {
-        const int ke = mx::KE(n), nb = ke + mx::KO(n);
-        for (int t = threadIdx.x; t < 16 * nb * nb; t += blockDim.x) {
-            const int rq = t / (16 * nb), kq = (t >> 4) % nb, i = (t >> 2) & 3, q = t & 3;
-            const int row = (rq < ke ? 8 * rq : 8 * (rq - ke) + 1) + 2 * i, col = (kq < ke ? 8 * kq : 8 * (kq - ke) + 1) + 2 * q;
-            A[at + t] = row <= n && col <= n ? tb.Ad[mx::ABASE(n) + row * mx::AST(n) + col] : 0.0;
-        }
-        at += 16 * nb * nb;
+        const int len = 16 * (mx::KE(n) + mx::KO(n)) * (mx::KE(n) + mx::KO(n));
+        for (int t = threadIdx.x; t < len; t += blockDim.x) T.A[at + t] = mx::padded(tb.Ad, n, t);
+        at += len;
     }
     for (int i = threadIdx.x; i < H; i += blockDim.x) {
         int n, m;
         idx_nm(i, n, m);
         const int b = len_Ts(n - 1);
-        zin[i] = tb.zeta[b + m];
-        zoh[i] = 0.5 * tb.zeta[b + m * (n + 1)];
-        ein[i] = tb.eta[b + m];
-        eoh[i] = 0.5 * tb.eta[b + m * (n + 1)];
-        Mt[i] = tb.Mt[i];
-        Lt[i] = tb.Lt[i];
+        T.zin[i] = tb.zeta[b + m];
+        T.zoh[i] = 0.5 * tb.zeta[b + m * (n + 1)];
+        T.ein[i] = tb.eta[b + m];
+        T.eoh[i] = 0.5 * tb.eta[b + m * (n + 1)];
+        T.Mt[i] = tb.Mt[i];
+        T.Lt[i] = tb.Lt[i];
     }
-    double* i0 = tf + 2 * NS;
-    for (int i = threadIdx.x; i < 2 * NS; i += blockDim.x) tf[i] = tb.tfac[i];
+    for (int i = threadIdx.x; i < 2 * NS; i += blockDim.x) T.tf[i] = tb.tfac[i];
     for (int n = threadIdx.x; n < NS; n += blockDim.x) {
-        i0[2 * n] = 1.0 / tb.Mt[nh(n - 1)];
-        i0[2 * n + 1] = 1.0 / tb.Lt[nh(n - 1)];
+        T.i0[2 * n] = 1.0 / tb.Mt[nh(n - 1)];
+        T.i0[2 * n + 1] = 1.0 / tb.Lt[nh(n - 1)];
     }
     __syncthreads();
-    double* wl = lds + mx_shared_doubles<CAP>() + (size_t)wave_id() * mx_wave_doubles<CAP, LH>();
-    const mx::Wave W{wl + NC * H, wl + NC * H + 2 * BP * NS, wl, wl + NC * H + 4 * BP * NS};
-    const mx::Tabs T{A, zin, zoh, ein, eoh, Mt, Lt, tf, i0};
+    const mx::Wave W = mx::wave<CAP, LH>(lds + mx::shared_doubles<CAP>() + (size_t)wave_id() * mx::wave_doubles<CAP, LH>());
     const int64_t HE4 = 4 * (int64_t)nh(PE);
     const int lane = lane_id();
     int pmax = 0, okf = 1;

@@ -1,13 +1,16 @@
 // Lane-by-lane CPU emulation of the matrix-core M2L engine (fastmultipole_amd/csrc/m2l_mx.hpp).
 // Test infrastructure: the engine's source is compiled here with a backend whose per-lane values are
 // arrays of 64 doubles, whose cross-lane moves are permutations of those arrays, and whose MFMA is
-// v_mfma_f64_16x16x4f64's product with its lane layout (lane l supplies A(l % 16, l / 16) and
-// B(l / 16, l % 16) and holds D(l / 16 + 4 r, l % 16) in element r). tests/test_m2l_mx_emul.py compares
-// the result with the oracle's multipole_to_local.
+// v_mfma_f64_4x4x4_4b_f64's product with its lane layout (four blocks; lane l supplies A(l % 4, l / 16) and
+// B(l / 16, l % 4) of block (l % 16) / 4 and holds its D(l / 16, l % 4)). The tables and the wavefront's
+// scratch lie in one array in the order of the GPU's LDS, NaN where nothing has been written, so a read of
+// anything but a written double shows. tests/test_m2l_mx_emul.py compares the result with the
+// oracle's multipole_to_local.
 #include <array>
 #include <cmath>
 #include <cstdint>
 #include <cstring>
+#include <limits>
 #include <vector>
 
 #include "../fastmultipole_amd/csrc/m2l_mx.hpp"
@@ -32,9 +35,6 @@ struct CpuB {
         std::array<double, W> v;
         V() { v.fill(0.0); }
         V(double x) { v.fill(x); }
-    };
-    struct V4 {
-        V r[4];
     };
     struct PV {
         std::array<const double*, W> v;
@@ -88,8 +88,6 @@ struct CpuB {
         return r;
     }
     static V perm1(const V& a) { return from(a, [](int i) { return i ^ 1; }); }
-    static V perm2(const V& a) { return from(a, [](int i) { return i ^ 2; }); }
-    static V perm3(const V& a) { return from(a, [](int i) { return i ^ 3; }); }
     static V bperm(const V& a, const I& src) {
         V r;
         for (int i = 0; i < W; ++i) r.v[i] = a.v[src.v[i] & 63];
@@ -117,17 +115,15 @@ struct CpuB {
         for (int i = 0; i < W; ++i) r.v[i] = a.v[(i & ~(NC - 1)) + j];
         return r;
     }
-    static V4 zero4() { return V4{}; }
-    static V get4(const V4& a, int r) { return a.r[r]; }
-    static void set4(V4& a, int r, const V& x) { a.r[r] = x; }
-    static void mfma(const V& a, const V& b, V4& d) {
-        for (int r = 0; r < 4; ++r)
-            for (int l = 0; l < W; ++l) {
-                const int i = l / 16 + 4 * r, j = l % 16;
-                double s = d.r[r].v[l];
-                for (int kk = 0; kk < 4; ++kk) s = std::fma(a.v[16 * kk + i], b.v[16 * kk + j], s);
-                d.r[r].v[l] = s;
-            }
+    static V mfma4(const V& a, const V& b, const V& d) {
+        V r;
+        for (int l = 0; l < W; ++l) {
+            const int i = l / 16, blk = (l % 16) / 4;   // D(i, j) of block blk: A of the block's lanes with l % 4 = i
+            double s = d.v[l];
+            for (int k = 0; k < 4; ++k) s = std::fma(a.v[16 * k + 4 * blk + i], b.v[16 * k + l % 16], s);
+            r.v[l] = s;
+        }
+        return r;
     }
     static bool any(const M& m) {
         for (int i = 0; i < W; ++i)
@@ -160,9 +156,9 @@ struct CpuB {
         for (int i = 0; i < W; ++i) r.v[i] = base + js.v[i] * stride;
         return r;
     }
-    static V gldp(const PV& p, const I& idx, const M& ok) {
+    static V gldp(const PV& p, const I& idx) {
         V r;
-        for (int i = 0; i < W; ++i) r.v[i] = ok.v[i] ? p.v[i][idx.v[i]] : 0.0;
+        for (int i = 0; i < W; ++i) r.v[i] = p.v[i][idx.v[i]];
         return r;
     }
     static V lds(const double* p, const I& idx) {
@@ -230,46 +226,46 @@ inline M operator!(const M& a) {
 inline M operator&&(const M& a, bool b) { return a && M(b); }
 inline M operator||(const M& a, bool b) { return a || M(b); }
 
-struct HostTabs {
-    std::vector<double> A, zin, zoh, ein, eoh, Mt, Lt, tf, i0;
-    explicit HostTabs(int cap) {
-        using namespace fmmhip::tabh;
-        std::vector<double> Hs, z, e;
-        host_Hs(Hs, cap);
-        host_mags(z, e, cap);
-        host_power_norms(Mt, Lt, cap);
-        A = host_dense_A(Hs, cap);
-        tf = host_test_factorials(cap);
-        const int H = nh(cap);
-        zin.resize(H); zoh.resize(H); ein.resize(H); eoh.resize(H);
-        i0.resize(2 * (cap + 1));
-        for (int n = 0; n <= cap; ++n) {
-            i0[2 * n] = 1.0 / Mt[nh(n - 1)];
-            i0[2 * n + 1] = 1.0 / Lt[nh(n - 1)];
+template <int CAP>
+void fill_tables(const fmmhip::mx::Tabs& T) {
+    using namespace fmmhip::tabh;
+    std::vector<double> Hs, z, e, Mt, Lt;
+    host_Hs(Hs, CAP);
+    host_mags(z, e, CAP);
+    host_power_norms(Mt, Lt, CAP);
+    const std::vector<double> A = host_dense_A(Hs, CAP), tf = host_test_factorials(CAP);
+    for (int n = 0, i = 0, at = 0; n <= CAP; ++n) {
+        const int len = fmmhip::mx::PBASE(n + 1) - fmmhip::mx::PBASE(n);
+        for (int t = 0; t < len; ++t) T.A[at + t] = fmmhip::mx::padded(A.data(), n, t);
+        at += len;
+        for (int m = 0; m <= n; ++m, ++i) {
+            const int b = len_Ts(n - 1);
+            T.zin[i] = z[b + m];
+            T.zoh[i] = 0.5 * z[b + m * (n + 1)];
+            T.ein[i] = e[b + m];
+            T.eoh[i] = 0.5 * e[b + m * (n + 1)];
+            T.Mt[i] = Mt[i];
+            T.Lt[i] = Lt[i];
         }
-        for (int n = 0, i = 0; n <= cap; ++n)
-            for (int m = 0; m <= n; ++m, ++i) {
-                const int b = len_Ts(n - 1);
-                zin[i] = z[b + m];
-                zoh[i] = 0.5 * z[b + m * (n + 1)];
-                ein[i] = e[b + m];
-                eoh[i] = 0.5 * e[b + m * (n + 1)];
-            }
+        T.tf[2 * n] = tf[2 * n];
+        T.tf[2 * n + 1] = tf[2 * n + 1];
+        T.i0[2 * n] = 1.0 / Mt[nh(n - 1)];
+        T.i0[2 * n + 1] = 1.0 / Lt[nh(n - 1)];
     }
-    fmmhip::mx::Tabs view() const {
-        return {A.data(), zin.data(), zoh.data(), ein.data(), eoh.data(), Mt.data(), Lt.data(), tf.data(), i0.data()};
-    }
-};
+}
 
-template <int CAP, bool LH>
+template <int CAP, bool LH, bool ERR>
 int run(int P, int kind, int relative, double eps, int BE, const double* tg, int nsrc, const double* sg,
-        const double* sex, int64_t he4, double* out, int32_t* orders, int* pmax, int* ok) {
-    using E = fmmhip::mx::Engine<CpuB, CAP, LH>;
-    static const HostTabs tabs(CAP);
-    const fmmhip::mx::Tabs T = tabs.view();
-    std::vector<double> eim(E::BP * E::NS * 2), cs(E::BP * E::NS * 2), acc(E::NC * fmmhip::mx::mnh(CAP), 0.0),
-        F(E::BP * E::NF);
-    fmmhip::mx::Wave Wv{eim.data(), cs.data(), acc.data(), F.data()};
+        const double* sex, int64_t he4, const int32_t* perm, double* out, int32_t* orders, int* pmax, int* ok) {
+    using E = fmmhip::mx::Engine<CpuB, CAP, LH, ERR>;
+    // the GPU's LDS of a workgroup of one wavefront, and as much again of what another wavefront has not written yet
+    constexpr int shared = fmmhip::mx::shared_doubles<CAP>(), wave = fmmhip::mx::wave_doubles<CAP, LH>();
+    std::vector<double> lds(shared + 2 * wave, std::numeric_limits<double>::quiet_NaN());
+    const fmmhip::mx::Tabs T = fmmhip::mx::tabs<CAP>(lds.data());
+    fill_tables<CAP>(T);
+    const fmmhip::mx::Wave Wv = fmmhip::mx::wave<CAP, LH>(lds.data() + shared);
+    double* acc = Wv.acc;
+    for (int i = 0; i < E::NC * fmmhip::mx::mnh(CAP); ++i) acc[i] = 0.0;
     fmmhip::mx::Box X;
     for (int d = 0; d < 3; ++d) { X.tc[d] = tg[3 + d]; X.tbox[d] = tg[11 + d]; }
     X.r_l = tg[7];
@@ -281,7 +277,7 @@ int run(int P, int kind, int relative, double eps, int BE, const double* tg, int
     for (int i = 0; i < nsrc; ++i) ms[i] = i;
     int pm = 0, okf = 1;
     for (int b0 = 0; b0 < nsrc; b0 += E::BP)
-        E::batch(T, Wv, X, fmmhip::mx::Batch{ms.data(), nullptr, b0, std::min(E::BP, nsrc - b0), orders}, sg, 15, 0, sex, he4,
+        E::batch(T, Wv, X, fmmhip::mx::Batch{ms.data(), perm, b0, std::min(E::BP, nsrc - b0), orders}, sg, 15, 0, sex, he4,
                  pm, okf);
     const int H = fmmhip::mx::mnh(P);
     for (int i = 0; i < H; ++i)
@@ -293,14 +289,13 @@ int run(int P, int kind, int relative, double eps, int BE, const double* tg, int
 
 }  // namespace
 
+// perm: processing order of the list (null: list order)
 extern "C" int mx_emul_m2l(int LH, int cap, int P, int kind, int relative, double eps, int BE, const double* tgeom,
-                           int nsrc, const double* sgeoms, const double* sexp, int64_t he4, double* out, int32_t* orders,
-                           int* pmax, int* ok) {
-#define MX_CASE(C)                                                                                                   \
-    if (cap == C)                                                                                                    \
-        return LH ? run<C, true>(P, kind, relative, eps, BE, tgeom, nsrc, sgeoms, sexp, he4, out, orders, pmax, ok)  \
-                  : run<C, false>(P, kind, relative, eps, BE, tgeom, nsrc, sgeoms, sexp, he4, out, orders, pmax, ok);
-    MX_CASE(8) MX_CASE(20)
-#undef MX_CASE
-    return -1;
+                           int nsrc, const double* sgeoms, const double* sexp, int64_t he4, const int32_t* perm, double* out,
+                           int32_t* orders, int* pmax, int* ok) {
+    constexpr int K = MX_CAP;   // one order cap per library (compiled side by side)
+    if (cap != K) return -1;
+#define MX_RUN(L, E) run<K, L, E>(P, kind, relative, eps, BE, tgeom, nsrc, sgeoms, sexp, he4, perm, out, orders, pmax, ok)
+    return kind ? (LH ? MX_RUN(true, true) : MX_RUN(false, true)) : (LH ? MX_RUN(true, false) : MX_RUN(false, false));
+#undef MX_RUN
 }
