@@ -68,6 +68,32 @@ def test_chunked_lists_match_the_wavefront_engine(p, kernel, monkeypatch):
         assert np.abs(outs["mx"][:, lo:hi] - ref).max() <= 1e-11 * max(np.abs(ref).max(), 1e-300)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("kernel", [_lib.POINT_SOURCE, _lib.POINT_VORTEX], ids=["source", "vortex"])
+@pytest.mark.parametrize("p,tol", [(8, 1e-3), (12, 1e-5), (16, 1e-6), (20, 1e-8)])
+def test_chunked_error_controlled_lists_match_the_wavefront_engine(p, tol, kernel, monkeypatch):
+    """Orders chosen per interaction, lists longer than a chunk, processed in an order of their own. The engines' test values
+    agree to a few ulps, so every order is the same (a tolerance within an ulp's reach of one is not met by 1e5 tests)."""
+    rows = W.plummer_sources(2600, seed=11) if kernel == _lib.POINT_SOURCE else W.uniform_vortices(2600, seed=11)
+    S = CHUNK[min(c for c in CHUNK if c >= p)] * (1 if kernel == _lib.POINT_VORTEX else 2)
+    outs, orders = {}, {}
+    for engine in ("mx", "wave"):
+        monkeypatch.setenv("FMMHIP_M2L_KERNEL", engine)
+        ev = F.Evaluation()
+        ev.set_systems(kernel, None, rows)
+        ev.fmm(F.make_options(expansion_order=p, leaf_size_source=12, multipole_acceptance=0.6, scalar_potential=True,
+                              gradient=True, hessian=True, error_tolerance=F.PowerRelativeGradient(tol)))
+        outs[engine], orders[engine] = ev.targets(), ev.m2l_orders()
+        lens = np.bincount(ev.list(0)[:, 0])
+        ev.close()
+    assert lens.max() > 2 * S
+    np.testing.assert_array_equal(orders["mx"], orders["wave"])
+    assert len(np.unique(orders["mx"])) > 2
+    for lo, hi in ((3, 4), (4, 7), (7, 16)):
+        ref = outs["wave"][:, lo:hi]
+        assert np.abs(outs["mx"][:, lo:hi] - ref).max() <= 1e-11 * max(np.abs(ref).max(), 1e-300)
+
+
 def _free_bytes():
     free, total = ctypes.c_size_t(), ctypes.c_size_t()
     assert _lib.load().hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0   # the runtime the library is linked to
