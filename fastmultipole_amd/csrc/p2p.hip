@@ -276,13 +276,16 @@ __device__ inline double rinv_guarded(double r2) {
     return __longlong_as_double((long long)(((uint64_t)hi << 32) | (bits & 0xffffffffull)));
 }
 
-// 1/r of two pairs of the FP64 point source, 0 for a coincident pair. The kernel is bound by vector issue (4M Plummer
-// sphere: 97 % of the cycles). The estimate is the FP32 unit's: the conversions there and back and its reciprocal square
-// root take under two issue slots, v_rsq_f64 four, and where every r^2 of the wavefront is a normal float (tested for
-// both pairs at once, in place of the zero tests and their selects) none is zero. One third-order step takes
+// 1/r of two pairs of the FP64 point source's potential, 0 for a coincident pair. The kernel is bound by vector issue (4M
+// Plummer sphere: 97 % of the cycles). The estimate is the FP32 unit's: the conversions there and back and its reciprocal
+// square root take under two issue slots, v_rsq_f64 four, and where every r^2 of the wavefront is a normal float (tested
+// for both pairs at once, in place of the zero tests and their selects) none is zero. One third-order step takes
 // |e| <= 2^-22 to 2^-66. Other distances (coincident bodies, r below 1e-19 or above 1e19) take v_rsq_f64 and the zero
-// test. 89 -> 84 ms for that sphere's 1.03e11 pairs. The other kernels, at fewer wavefronts per SIMD, lose more to the
-// branch than the estimate gains (45k vortex ring 2.93 -> 3.18 ms) and keep v_rsq_f64.
+// test. 89 -> 84 ms for that sphere's 1.03e11 pairs, 12.4 -> 11.9 ms for 1M bodies in a cube; launches with few
+// wavefronts per SIMD, which the branch leaves waiting, lose (10k in a cube 0.533 -> 0.560 ms). Without the potential the
+// zero test is one select, and the estimate gains at most 1 % (1M 11.5 -> 11.4 ms) where it loses 19 % (10k 0.480 ->
+// 0.570 ms); the other kernels, at fewer wavefronts per SIMD, lose more to the branch than it gains (45k vortex ring
+// 2.93 -> 3.18 ms). All of these keep v_rsq_f64.
 __device__ inline double rinv_refine(double r2, double y) {
     const double e = fma(-r2 * y, y, 1.0);
     return fma(y * e, fma(e, 0.375, 0.5), y);
@@ -294,7 +297,6 @@ __device__ inline uint64_t not_normal(float x) {
     asm("v_cmp_class_f32 %0, %1, %2" : "=s"(m) : "v"(x), "v"(0x3ff & ~0x100));
     return m;
 }
-template <bool FULL>
 __device__ inline void rinv_pairs(double r2a, double r2b, double& ria, double& rib) {
     const float fa = (float)r2a, fb = (float)r2b;
     ria = (double)__builtin_amdgcn_rsqf(fa);
@@ -302,8 +304,8 @@ __device__ inline void rinv_pairs(double r2a, double r2b, double& ria, double& r
     ria = rinv_refine(r2a, ria);
     rib = rinv_refine(r2b, rib);
     if (__builtin_expect((not_normal(fa) | not_normal(fb)) != 0ull, 0)) {
-        ria = rinv_guarded<FULL>(r2a);
-        rib = rinv_guarded<FULL>(r2b);
+        ria = rinv_guarded<true>(r2a);
+        rib = rinv_guarded<true>(r2b);
     }
 }
 
@@ -325,12 +327,11 @@ __device__ inline void p2p_source_f64(const double* __restrict__ q, double xa, d
         if (r2a > 0.0) pair_eval<KERNEL, PS, GS, HS, double>(dxa, dya, dza, r2a, rinv_f64(r2a), gs, a);
         if (r2b > 0.0) pair_eval<KERNEL, PS, GS, HS, double>(dxb, dyb, dzb, r2b, rinv_f64(r2b), gs, b);
     } else {
-        constexpr bool FULL = KERNEL == FMMHIP_POINT_SOURCE && PS;
         double ria, rib;
-        if constexpr (KERNEL == FMMHIP_POINT_SOURCE) rinv_pairs<FULL>(r2a, r2b, ria, rib);
+        if constexpr (KERNEL == FMMHIP_POINT_SOURCE && PS) rinv_pairs(r2a, r2b, ria, rib);
         else {
-            ria = rinv_guarded<FULL>(r2a);
-            rib = rinv_guarded<FULL>(r2b);
+            ria = rinv_guarded<false>(r2a);
+            rib = rinv_guarded<false>(r2b);
         }
         pair_eval<KERNEL, PS, GS, HS, double>(dxa, dya, dza, r2a, ria, gs, a);
         pair_eval<KERNEL, PS, GS, HS, double>(dxb, dyb, dzb, r2b, rib, gs, b);
