@@ -950,8 +950,8 @@ static void fmm_run(Run& R, bool estimate_pass) {
     // The passes are split over OpenMP threads the way the reference's multithreaded drivers split
     // them (src/fmm.jl:57-93, 348-438, 492-598, 642-757): by target leaf (nearfield, L2P), by source
     // leaf (P2M), by parent branch within a level (M2M), by target branch (M2L) and by child branch
-    // within a level (L2L). Every expansion and target value is written by one thread and accumulates
-    // its terms in the serial order, so results are bit-identical for any thread count.
+    // within a level (L2L). Every expansion and target value is written by one thread at a time and
+    // accumulates its terms in the serial order, so results are bit-identical for any thread count.
     // target ranges of the target-sorted lists
     auto runs_of = [](const std::vector<std::array<int32_t, 2>>& L) {
         std::vector<size_t> r;
@@ -960,35 +960,33 @@ static void fmm_run(Run& R, bool estimate_pass) {
         r.push_back(L.size());
         return r;
     };
-    // nearfield (src/fmm.jl:3-40)
-    if (R.kinds.empty()) {
-        const std::vector<size_t> rd = runs_of(R.direct);
-        const int64_t nr = (int64_t)rd.size() - 1;
+    // nearfield (src/fmm.jl:3-40). SelfTuning's direct targets can lie inside one another (pairs of branches that are not
+    // leaves): the targets of one tree level at a time, which are disjoint, ancestors first as in the sorted list
+    const std::vector<size_t> rd = runs_of(R.direct);
+    auto nearfield = [&](auto&& pair) {
+        size_t g0 = 0;
+        for (size_t lv = 0; lv < R.tt.levels.size(); ++lv) {
+            size_t g1 = g0;
+            while (g1 + 1 < rd.size() && R.direct[rd[g1]][0] <= R.tt.levels[lv][1]) ++g1;
 #pragma omp parallel for schedule(dynamic, 1)
-        for (int64_t g = 0; g < nr; ++g)
-            for (size_t k = rd[g]; k < rd[g + 1]; ++k) {
-                const auto& pr = R.direct[k];
-                const OBranch& s = R.st.branches[pr[1]];
-                const OBranch& t = R.tt.branches[pr[0]];
-                user_direct(R.kind, R.tt.buffer.data(), t.first, t.n_bodies, R.st.buffer.data(), dpb, s.first, s.n_bodies,
-                            o.PS, o.GS, o.HS);
-            }
-    }
+            for (int64_t g = (int64_t)g0; g < (int64_t)g1; ++g)
+                for (size_t k = rd[g]; k < rd[g + 1]; ++k) pair(R.tt.branches[R.direct[k][0]], R.st.branches[R.direct[k][1]]);
+            g0 = g1;
+        }
+    };
+    if (R.kinds.empty())
+        nearfield([&](const OBranch& t, const OBranch& s) {
+            user_direct(R.kind, R.tt.buffer.data(), t.first, t.n_bodies, R.st.buffer.data(), dpb, s.first, s.n_bodies, o.PS,
+                        o.GS, o.HS);
+        });
     // several systems: each source system in turn over the whole direct list, with its own kernel
-    for (size_t is = 0; is < R.kinds.size(); ++is) {
-        const std::vector<size_t> rd = runs_of(R.direct);
-        const int64_t nr = (int64_t)rd.size() - 1;
-#pragma omp parallel for schedule(dynamic, 1)
-        for (int64_t g = 0; g < nr; ++g)
-            for (size_t k = rd[g]; k < rd[g + 1]; ++k) {
-                const auto& pr = R.direct[k];
-                const OBranch& t = R.tt.branches[pr[0]];
-                int64_t s0, sn;
-                system_range(R, R.st.branches[pr[1]], is, s0, sn);
-                user_direct(R.kinds[is], R.tt.buffer.data(), t.first, t.n_bodies, R.st.buffer.data(), dpb, s0, sn,
-                            o.PS, o.GS, o.HS);
-            }
-    }
+    for (size_t is = 0; is < R.kinds.size(); ++is)
+        nearfield([&](const OBranch& t, const OBranch& s) {
+            int64_t s0, sn;
+            system_range(R, s, is, s0, sn);
+            user_direct(R.kinds[is], R.tt.buffer.data(), t.first, t.n_bodies, R.st.buffer.data(), dpb, s0, sn, o.PS, o.GS,
+                        o.HS);
+        });
     // upward pass: P2M (src/bodytomultipole.jl:19-26) then M2M (src/fmm.jl:262-284)
     const int64_t nsl = (int64_t)R.st.leaf_index.size();
 #pragma omp parallel

@@ -302,3 +302,23 @@ def test_source_dipole_panel_fmm_is_source_plus_dipole_fmm(quads):
     for lo, hi in ((3, 4), (4, 7)):
         err = np.abs(got[:, lo:hi] - ref[:, lo:hi]).max() / np.abs(ref[:, lo:hi]).max()
         assert err < 1e-6, (lo, err)
+
+
+@pytest.mark.parametrize("method", [O.METHOD_SELFTUNING, O.METHOD_SELFTUNING_TREESTOP])
+def test_results_do_not_depend_on_the_thread_count(method):
+    """SelfTuning's direct targets lie inside one another: a thread per target would update a body from two threads."""
+    b = W.uniform_sources(5000, seed=700)
+
+    def run(threads):
+        O.threads(threads)
+        r = O.Run(O.KIND_SOURCE, b[:, :3], b, p=1, leaf_size_source=24, method=method, multipole_acceptance=0.45,
+                  scalar_potential=True, hessian=True).fmm()
+        return r.targets()
+
+    default = O.threads()
+    try:
+        want = run(1)
+        for _ in range(20):
+            np.testing.assert_array_equal(run(64), want)
+    finally:
+        O.threads(default)
