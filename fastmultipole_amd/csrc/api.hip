@@ -486,7 +486,7 @@ static void eval_core(Eval& E, const fmmhip_options& o, fmmhip_stats* stats, boo
                 LAUNCH_CHECK();
             }
             run_m2l(F, E.tt, E.st, E.tt, E.lists, p, LH, o.error_kind, o.error_relative != 0, o.error_tolerance,
-                    o.error_bonus != 0, o.precision, nullptr, nullptr);
+                    o.error_bonus != 0, o.precision);
             if (batch) {
                 int32_t pmax = 0, ok = 1;
                 if (E.lists.n_m2l_targets > 0) {

@@ -1984,7 +1984,7 @@ static M2LEngine m2l_engine() {
 }
 
 void run_m2l(Context& C, const Tree& tt, Tree& st, Tree& tt_dst, Lists& Ls, int p, bool LH, int err_kind, bool err_rel,
-             double eps, bool BE, int precision, int32_t* pmax, int32_t* success) {
+             double eps, bool BE, int precision) {
     (void)precision;
     (void)tt;
     ensure_tables(C, p);
@@ -2021,12 +2021,6 @@ void run_m2l(Context& C, const Tree& tt, Tree& st, Tree& tt_dst, Lists& Ls, int 
             run(C, p, p, M2L_PASS_ALL, Ls, st, tt_dst, E, flags.data(), tb);
         }
     }
-    if (!pmax) return;   // no read-back: the launch sequence stays free of host synchronisation (graph capture)
-    int32_t h[2];
-    HIP_CHECK(hipMemcpyAsync(h, flags.data(), sizeof(h), hipMemcpyDeviceToHost, C.stream));
-    HIP_CHECK(hipStreamSynchronize(C.stream));
-    *pmax = h[0];
-    *success = h[1];
 }
 
 __global__ void k_fill_zero(double* __restrict__ p, int64_t n) {

@@ -524,7 +524,7 @@ static void fgs_farfield(Eval& E, FgsState& F) {
     ensure_tables(C, p);
     run_p2m(C, E.kernel, E.st, p);
     run_m2m(C, E.st, p, false);
-    run_m2l(C, E.tt, E.st, E.tt, E.lists, p, false, FMMHIP_ERR_NONE, false, 0.0, true, FMMHIP_FP64, nullptr, nullptr);
+    run_m2l(C, E.tt, E.st, E.tt, E.lists, p, false, FMMHIP_ERR_NONE, false, 0.0, true, FMMHIP_FP64);
     run_l2l(C, E.tt, p, false);
     run_l2p(C, E.tt, E.tout.data(), E.nt, p, false, true, true, false);
 }

@@ -290,9 +290,9 @@ static constexpr int64_t M2L_PART_BYTES = (int64_t)2 << 30;
 // sbr: the source tree's branches with one system's leaf ranges (several systems in one tree), or null
 void run_p2m(Context& C, int kernel, Tree& st, int p, const Branch* sbr = nullptr);
 void run_m2m(Context& C, Tree& st, int p, bool LH);
-// pmax / success null: no read-back of the launch's largest order and tolerance flag (no host synchronisation)
+// leaves the largest order used and whether every tolerance was met in the context's m2l_flags (no host synchronisation)
 void run_m2l(Context& C, const Tree& tt, Tree& st_src, Tree& tt_dst, Lists& L, int p, bool LH, int err_kind,
-             bool err_rel, double eps, bool BE, int precision, int32_t* pmax, int32_t* success);
+             bool err_rel, double eps, bool BE, int precision);
 void run_l2l(Context& C, Tree& tt, int p, bool LH);
 // zeroes n doubles with a kernel (graph-capturable, unlike hipMemsetAsync)
 void fill_zero(Context& C, double* p, size_t n);

@@ -104,13 +104,13 @@ static size_t mx_lds_bytes(int nw) {
 
 // Work items. A target box's list entries are cut into chunks of S (the last one shorter), and a wavefront takes one
 // chunk at a time: with a wavefront per box the launch lasted as long as its longest list (45k ring at cap 20, 24,644
-// interactions in 1,400 boxes: 4.05 ms, when its 6,500 batches over 1024 wavefronts are 0.5 ms of work). Chunk c of
+// interactions in 1,400 boxes: 4.05 ms; 0.8 ms in chunks). Chunk c of
 // box b has slot l0 / S + b + c, l0 the box's first list entry: chunks of different boxes never share a slot
 // (ceil(len / S) <= floor(l1 / S) - floor(l0 / S) + 1), and the last slot is known on the host without a scan.
 // A box of one chunk is added to its target's expansion by the wavefront that holds it; the chunks of the others go to
 // `part` and k_m2l_mx_sum adds them in chunk order. S depends on the cap alone, never on the size of the problem, so a
-// box's sum is the same to the last bit whatever is evaluated beside it. S is a few batches: a chunk's partial
-// expansion (7.4 KB at cap 20) is written and read once per S interactions, 0.3 ms of the 1M ring's 30 ms.
+// box's sum is the same to the last bit whatever is evaluated beside it. S is one batch up to cap 12 and two above: a
+// chunk's partial expansion (7.4 KB at cap 20) is written and read once per S interactions, 1.2 GB of the 1M ring's 32 GB.
 __host__ __device__ inline int64_t mx_first_slot(int64_t l0, int64_t box, int S) { return l0 / S + box; }
 
 // The partial expansions take M2L_PART_BYTES at most. The slots of larger launches are taken in passes: the pass from w0 to
@@ -141,7 +141,9 @@ __device__ inline int mx_box_of(const int64_t* __restrict__ m2l_offsets, int n_b
 // cores, the rest waits on LDS and the gathered expansions (4M Plummer sphere, order 8, 22.9M interactions: 31.9 -> 9.0 ms,
 // 2.5e9 translations/s). At cap 16 and 20 the local expansion fills the registers (204 and 300 per lane; beyond 256
 // they move through accumulation registers), one wavefront per SIMD, LDS latency exposed (300k sphere, order 16:
-// 7.6 -> 3.7 ms, 6.3 ms when forced to two wavefronts; 1M ring, orders to 20: 28 -> 20.3 ms).
+// 7.6 -> 3.7 ms, 6.3 ms when forced to two wavefronts; 1M ring, orders to 20: 28 -> 20.3 ms). What does not fit 512 registers
+// goes to scratch memory: with the tests and two potentials 1.3 KB a lane at cap 20, about 23 of the 32 GB that the 1M
+// ring's launch moves, and 0.3 KB at cap 16; 0.1 to 0.6 KB at cap 12, held to 256 for its two wavefronts.
 template <int CAP, bool LH, int NW, bool ERR>
 __global__ __launch_bounds__(64 * NW, CAP <= 12 ? 2 : 1) void k_m2l_mx(const int32_t* __restrict__ m2l_targets,
                                                     const int64_t* __restrict__ m2l_offsets,
