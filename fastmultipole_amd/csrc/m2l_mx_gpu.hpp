@@ -113,9 +113,10 @@ static size_t mx_lds_bytes(int nw) {
 // chunk's partial expansion (7.4 KB at cap 20) is written and read once per S interactions, 1.2 GB of the 1M ring's 32 GB.
 __host__ __device__ inline int64_t mx_first_slot(int64_t l0, int64_t box, int S) { return l0 / S + box; }
 
-// The partial expansions take M2L_PART_BYTES at most. The slots of larger launches are taken in passes: the pass from w0 to
-// w1 takes every chunk of the boxes whose first slot lies in it, up to `span` slots past w1 (a list holds a source branch
-// once, so its chunks are no more than n_branches / S), and k_m2l_mx_sum adds them before the next pass. A box is summed
+// The partial expansions take M2L_PART_BYTES at most (or two of the longest lists possible, if that is more: from about 0.6M
+// branches at order 20). The slots of larger launches are taken in passes: the pass from w0 to w1 takes every chunk of the
+// boxes whose first slot lies in it, up to `span` slots past w1 (a list holds a source branch once, so its chunks are no
+// more than n_branches / S), and k_m2l_mx_sum adds them before the next pass. A box is summed
 // whole in one pass, so its sum does not depend on where the passes end. One pass for 4M bodies at order 8 (1.1 GB) or
 // the 1M ring at order 20 (1.0 GB); without a bound 2.5M uniform vortices at order 20 (37M interactions) took 20.7 GiB,
 // and 428 ms against 430 ms in ten passes.

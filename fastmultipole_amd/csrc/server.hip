@@ -68,8 +68,9 @@ double footprint_bytes(const fmmhip_request& r) {
         // about 150 interactions per box (measured: 135 of uniform sources at acceptance 0.4), a slot more than its full
         // chunks for each box, up to the workspace's bound; the buffer's slack of an eighth
         const bool lh = fmmhip::has_vector_potential(r.kernel);
-        const double slots = branches * (150.0 / fmmhip::m2l_chunk(p, lh) + 1.0);
-        b += 1.125 * std::min(slots * (lh ? 32.0 : 16.0) * H, (double)fmmhip::M2L_PART_BYTES);
+        const double chunk = fmmhip::m2l_chunk(p, lh), bytes = (lh ? 32.0 : 16.0) * H;
+        b += 1.125 * std::min(branches * (150.0 / chunk + 1.0) * bytes,
+                              std::max((double)fmmhip::M2L_PART_BYTES, 2.0 * branches / chunk * bytes));
     }
     if (fmmhip::is_panel(r.kernel)) b += 1.125 * n * 8.0 * fmmhip::panel_record_doubles(fmmhip::panel_vertices(r.kernel));
     if (r.kind == FMMHIP_REQUEST_SOLVE) b += n * leaf * 8.0 * 30.0 + n * 8.0 * 40.0;
